@@ -176,7 +176,10 @@ FA2_API int fa2_ablate_tail_schedule(int32_t batch, int32_t h_q, int32_t h_kv, i
  * with the kernel's own code (program_of and the dynamic tail's ticket rules, which are
  * __host__ __device__) on a device of `cus` CUs and `xcds` XCDs. The launch is fa2_attn_fwd's on
  * contiguous tensors of these sizes (n_kv = n_q) at block_m rows and the default tile, without
- * split-KV; static_order != 0 keeps the static order (FA2_ABLATE_STATIC_ORDER).
+ * split-KV; static_order != 0 keeps the static order (FA2_ABLATE_STATIC_ORDER). It is the general
+ * kernel's launch, except with static_order 2, which follows fa2_attn_fwd's choice of kernel: where
+ * that is the wave-split kernel, the programs are (row tile, batch, first query head of the KV
+ * head) of its workgroups, and info's unit chunk holds the rows of a row tile.
  * tail_private_pct is the share of each XCD's tail programs its own queue holds: -1 for the
  * library's (what fa2_attn_fwd launches), or 0..100 to plan another build's policy (the
  * FA2_TAIL_PRIVATE_PCT a variant build is compiled with). The dynamic tail's workgroups take

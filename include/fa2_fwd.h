@@ -97,6 +97,9 @@ FA2_API int fa2_attn_fwd(const void* q, const void* k, const void* v, void* out,
  *              that many pieces of whole K/V tiles (fewer if the key range is shorter), one
  *              workgroup each, and a second kernel merges the pieces. For grids too small
  *              to fill the GPU: few queries against a long K/V. fa2_num_splits() picks it.
+ *              At the default tiles (block_m 128), few rows per KV head and small grids run a
+ *              kernel whose workgroups share a row's keys among their waves; it takes at most
+ *              num_splits pieces, and fewer where those already reach every CU.
  *   workspace  device memory, 256-byte aligned, owned by the caller and untouched until the
  *              launch has run; may be NULL when num_splits == 1. It must hold at least
  *              fa2_workspace_bytes(batch, h_q, n_q, head_dim, num_splits) bytes (the split-KV
@@ -179,7 +182,8 @@ FA2_API size_t fa2_workspace_bytes_for(int32_t batch, int32_t h_q, int32_t h_kv,
 /*
  * fa2_num_splits - the split count fa2_attn_fwd_ex should use: 1 for causal launches and for
  * grids of at least num_cus workgroups; otherwise the smallest power of two that reaches it,
- * keeping at least 4 K/V tiles per split, at most 16. The grid it sizes is the
+ * keeping at least 4 K/V tiles per split, at most 16; or more where the kernel for few rows per KV
+ * head (at most 64) uses more. The grid it sizes is the
  * smaller of the packed and the unpacked GQA layouts, so the answer does not depend on the
  * packing decision and packed and unpacked launches stay equal bit for bit. Host policy only.
  */

@@ -1,0 +1,88 @@
+"""GPU parity of the wave-split kernel (csrc/attn_fwd_wavesplit.hpp): few rows per KV head and
+small grids at the default tiles. At the edges of its row tiles (32 and 64 rows), of its key tiles
+(32, 64, 128 keys by head_dim) and of the key groups' turns, against the oracle with the reference's
+rule, and against the general kernel on the same inputs (127 rows a program keep a call off the
+wave-split kernel): outputs that round the same attention differ by a few roundings, so by less
+than 2^-6 of a row of unit-variance values in bf16 and 2^-9 in fp16.
+"""
+
+import pytest
+import torch
+
+from attn_check import check_against_oracle, make_qkv
+from oracle import reference as ref
+
+pytestmark = pytest.mark.gpu
+
+LSE_ATOL = 1e-4  # tests/test_gpu_splitkv.py
+
+
+def _attention():
+    from fa2.kernel import attention
+    return attention
+
+
+def _check(q, k, v, causal):
+    attention = _attention()
+    out, lse = attention(q, k, v, causal=causal, return_lse=True)
+    assert torch.equal(out, attention(q, k, v, causal=causal))
+    check_against_oracle(q, k, v, causal, ours=out)
+    want = ref.naive_lse(q.double(), k.double(), None, causal=causal)
+    assert (lse.double() - want).abs().max().item() <= LSE_ATOL
+    general = attention(q, k, v, causal=causal, block_m=127, pack_gqa=False, num_splits=1)
+    ulp = 2.0 ** (-6 if q.dtype == torch.bfloat16 else -9)
+    assert (out.float() - general.float()).abs().max().item() <= ulp * v.float().abs().max().item()
+
+
+# rows per KV head (n_q * group) below, at and past 32 and 64; key counts at the edges of a tile and
+# of a round of the four key groups (128 / 256 / 512 keys), one and several splits
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("h_q,h_kv,n_q,n_kv", [
+    (8, 2, 1, 129), (8, 2, 8, 255), (8, 2, 8, 512), (28, 4, 1, 1537), (20, 4, 7, 300), (6, 2, 11, 193),
+    (8, 8, 32, 321), (4, 4, 33, 640), (8, 2, 16, 1000), (5, 1, 13, 4100), (2, 2, 64, 9000),
+    (8, 1, 1, 3000), (4, 4, 333, 1500), (8, 2, 65, 2048)])
+def test_full(dtype, D, h_q, h_kv, n_q, n_kv):
+    _check(*make_qkv(2, h_q, h_kv, n_q, n_kv, D, dtype), causal=False)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("B,h_q,h_kv,n", [
+    (1, 4, 4, 129), (2, 8, 2, 193), (1, 4, 1, 256), (3, 5, 1, 383), (1, 28, 4, 400), (1, 8, 2, 1000),
+    (2, 16, 16, 520), (1, 32, 8, 1030)])
+def test_causal(dtype, D, B, h_q, h_kv, n):
+    _check(*make_qkv(B, h_q, h_kv, n, n, D, dtype), causal=True)
+
+
+def test_many_units_and_strided_storage():
+    """More units than CUs, an odd unit count, and [B, N, H, D] storage."""
+    attention = _attention()
+    for causal, shape in ((False, (37, 16, 8, 2, 500, 64)), (False, (3, 12, 12, 512, 512, 64)),
+                          (True, (3, 12, 12, 512, 512, 64)), (False, (1, 16, 16, 512, 512, 128))):
+        q, k, v = make_qkv(*shape, torch.bfloat16)
+        want = attention(q, k, v, causal=causal)
+        check_against_oracle(q, k, v, causal, ours=want)
+        qs, ks, vs = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v))
+        assert torch.equal(attention(qs, ks, vs, causal=causal), want)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_scores_that_rise_and_extreme_keys(causal):
+    """Keys that grow along the sequence move every group's reference on every tile; a key row of
+    +/-inf or NaN makes the rows that see it NaN, as the general kernel does, and no other."""
+    attention = _attention()
+    q, k, v = make_qkv(1, 8, 2, 600, 600, 64, torch.float16)
+    ramp = torch.linspace(0.0, 6.0, 600, device=q.device)[:, None].half()
+    check_against_oracle(q, k + ramp * q[:, :2].mean(dim=2, keepdim=True), v, causal)
+    for bad in (float("inf"), float("nan")):
+        kb = k.clone()
+        kb[:, 1, 450] = bad
+        out = attention(q, kb, v, causal=causal)
+        general = attention(q, kb, v, causal=causal, block_m=127, pack_gqa=False, num_splits=1)
+        assert torch.equal(out[:, :4].isnan(), general[:, :4].isnan())
+        assert not out[:, :4].isnan().any()
+        if causal:
+            assert not out[:, 4:, :450].isnan().any()
+        if bad != bad:
+            assert out[:, 4:, 450 if causal else 0:].isnan().all()

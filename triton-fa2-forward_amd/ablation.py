@@ -158,16 +158,19 @@ def attention_ablate(q, k, v, causal=True, pack_gqa=False, **knobs):
     return out
 
 
-def table_free_launch(q, k, v, causal):
-    """fa2_attn_fwd at the default configuration: the product kernel without the key-norm table,
-    which is what `copy` must equal bit for bit."""
+def table_free_launch(q, k, v, causal, block_m=127):
+    """fa2_attn_fwd without the key-norm table. With 127 rows a program the library always runs the
+    general kernel (a small grid at the default 128 takes the wave-split kernel, which sums a row in
+    another order), and a row's arithmetic there does not depend on block_m: the result is the
+    general kernel's at its default tiles, bit for bit. block_m 128 is the product's own launch,
+    which `copy` must equal bit for bit."""
     import torch
 
     from fa2 import _lib
     from fa2.kernel import LOG2E
 
     out = torch.empty_like(q)
-    _lib.attn_fwd(q, k, v, out, causal, 1, 128, 0, LOG2E / math.sqrt(q.shape[3]),
+    _lib.attn_fwd(q, k, v, out, causal, 1, block_m, 0, LOG2E / math.sqrt(q.shape[3]),
                   torch.cuda.current_stream().cuda_stream)
     return out
 
@@ -239,7 +242,7 @@ def measure_shape(args, N):
     q, k, v = (t.to(dtype).cuda() for t in (q, k, v))
     flops = bench.attn_flops(args.batch, args.hq, N, N, args.head_dim, causal)
 
-    product = table_free_launch(q, k, v, causal)
+    product = table_free_launch(q, k, v, causal, block_m=128)
     shipped = attention(q, k, v, causal=causal)
     launchers = {"attention()": lambda: attention(q, k, v, causal=causal)}
     outputs = {}

@@ -17,6 +17,7 @@
 #include <mutex>
 #include <utility>
 
+#include "attn_fwd_common.hpp"
 #include "attn_fwd_launch.hpp"
 #include "fa2_fwd.h"
 
@@ -103,6 +104,85 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
   const double flops = 4.0 * batch * h_q * pairs * head_dim;
   const double kbytes = 2.0 * batch * h_kv * n_kv * head_dim;
   return kbytes > 0 && flops >= 16384.0 * kbytes && flops >= 137438953472.0;  // 2^37
+}
+
+// The kernel choice of a call at the default tiles: the wave-split kernel (attn_fwd_wavesplit.hpp)
+// with 32 * row_waves rows a workgroup and `splits` key ranges, or the general kernel
+// (row_waves 0). Independent of pack, as packed and unpacked calls must agree bit for bit.
+//
+// The wave-split kernel walks a row's keys with 4 / row_waves waves at once, which shortens a
+// launch that its longest key range bounds, but it stages K/V into LDS two or four times as often
+// per row, so a grid that fills the GPU belongs to the general kernel. Where the line lies was
+// measured on MI355X (us per launch in a graph, general kernel -> this one; w1 and w2 are the
+// workgroups at 32 and 64 rows; 256 CUs hold two of them each):
+//   * few rows (at most 64 per KV head, not causal), bound by reading K/V: bf16 H32/8 D128 one
+//     query of 32000 keys 50.5 -> 32.4, of 1000 10.1 -> 7.9, B16 4096 keys 59.9 -> 49.4, B16 with 16
+//     queries 62.2 -> 53.4, H28/4 D64 B8 5712 keys 53.4 -> 15.1 (the general kernel cannot pack a
+//     group of 7); B40 of 2000 keys 65.2 -> 67.8 is the one loss seen.
+//   * causal, one round of workgroups (D128 H8/2): N 512 12.5 -> 8.5, 1024 20.8 -> 11.5, 2048
+//     37.5 -> 20.9, 4096 (w2 512) 69.7 -> 55.1; H32/8 N 256 8.9 -> 7.4, 512 13.0 -> 10.7, 1024
+//     (w2 512) 22.7 -> 20.3, but 2048 (w2 1024) 45.8 -> 50.5. D64 H16 N 256 7.7 -> 5.7, 1024 16.0
+//     -> 9.3, 2048 (w2 512) 28.4 -> 20.7; B4 1024 (w2 1024) 19.9 -> 23.1. D32 H16 B2 N 2048 (w2
+//     1024; its small tiles let a CU hold four workgroups) 24.0 -> 20.0, B4 (w2 2048) 34.3 -> 36.6.
+//   * full, more rows: H16 D64 N 512 9.2 -> 6.3, 1024 (w2 256) 14.4 -> 11.3, 2048 (w2 512) 27.5 ->
+//     27.2; B2 H16 D64 333 x 1500 20.7 -> 14.0; H32/8 D128 64 x 2048 B4 23.4 -> 17.2. Every row
+//     tile reads its KV head's keys again, so past some thousand keys the general kernel and its
+//     split are better: H32/8 D128 128 x 4096 24.6 -> 26.3, D64 H16 256 x 8192 23.0 -> 29.8.
+//   * up to 128 keys (192 at head_dim 128, where tiles are small) there is little to share out:
+//     D128 H32/8 N 64 5.1 -> 6.5, N 128 6.7 -> 6.6, N 192 7.3 -> 7.3.
+struct KernelChoice {
+  int row_waves = 0, splits = 1;
+};
+KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64_t n_kv,
+                           int32_t head_dim, bool causal, int32_t block_m, int32_t bn, int cus,
+                           int max_splits) {
+  KernelChoice kc;
+  kc.splits = max_splits;  // the general kernel takes the count it is given
+  if (block_m != 128 || bn != default_block_n(head_dim)) return kc;
+  const int64_t rows = n_q * (h_q / h_kv), units = batch * h_kv;
+  if (n_kv <= (head_dim == 128 && (causal || rows > 32) ? 192 : 128)) return kc;
+  if (rows > (int64_t(1) << 22) || units > (int64_t(1) << 22)) return kc;  // (products below fit)
+  const int64_t w1 = (rows + 31) / 32 * units, w2 = (rows + 63) / 64 * units;
+  const bool small = head_dim <= 32;
+  // The splits of a launch of 32-row workgroups: doubled until one more doubling would pass one
+  // workgroup per CU or leave a wave without a tile, where a wave has tiles enough for the merge
+  // launch (~2 us) to pay: 7 of 32 keys x D128, or 14 where only one doubling fits. Measured (us at
+  // 1, 2, 4, 8, 16 splits; D128 H32/8, one query): B1 of 1000 keys (7.8 tiles a wave) 9.0 8.9 7.9
+  // 7.7 8.3, 4000 23.7 16.7 12.1 10.1 10.0; B4 4000 24.0 17.6 15.2 15.2 16.4; B12 1500 14.2 15.9
+  // 16.6, 4000 46.2 38.6 41.2; B16 1000 12.8 15.0, 4000 49.4 48.4 50.0; B24 4000 67.2 75.0 71.7. The
+  // 128-key tiles of D16 and D32 take about twice as long each: D16 MQA B4 2000 keys (3.9 tiles) 8.1
+  // 8.1 7.3 7.7 8.3.
+  auto take_splits = [&]() {
+    kc.splits = 1;
+    const int step = 4 * fa2::wave_split_block_n(head_dim, 1, false);
+    const int64_t tiles = n_kv / step;  // ... a wave walks without splits
+    const int64_t least = (4 * w1 <= cus ? 7 : 14) * (int64_t)step / (small ? 2 : 1);
+    if (n_kv >= least)
+      while (kc.splits * 2 <= max_splits && w1 * kc.splits * 2 <= cus && tiles / kc.splits >= 2)
+        kc.splits *= 2;
+  };
+  if (causal) {  // (num_splits is 1)
+    if (w1 <= cus || (w1 <= 2 * cus && n_kv >= 384))
+      kc.row_waves = 1;
+    else if (w2 <= (small ? 4 : 2) * cus && n_kv >= (head_dim == 128 ? 512 : 0))
+      kc.row_waves = 2;
+  } else if (rows <= 64) {
+    kc.row_waves = 1;
+    take_splits();
+  } else if (n_kv <= (head_dim == 128 ? 2048 : 4096)) {
+    if (w1 <= cus) {
+      kc.row_waves = 1;
+      take_splits();
+    } else if (w1 <= 2 * cus && n_kv >= (small ? 512 : 0)) {
+      // two workgroups on some CUs: 64 rows a workgroup where that still reaches every CU
+      kc.row_waves = 10 * w2 >= 9 * cus ? 2 : 1;
+      kc.splits = 1;
+    } else if (small && w2 <= 2 * cus && n_kv >= 512) {
+      kc.row_waves = 2;
+      kc.splits = 1;
+    }
+  }
+  return kc;
 }
 
 // Topology of a device as the program order uses it: log2 of its XCD count and its CU count.
@@ -404,6 +484,9 @@ void finish_tickets(TicketSet* set, bool launched) {
 using KernelLaunch = int (*)(int dtype, int di, const Params& p, int waves, int block_n,
                              bool causal, unsigned grid, hipStream_t s, int variant,
                              hipEvent_t stop);
+// ... and the wave-split kernel (32 * row_waves rows a workgroup).
+using SplitLaunch = int (*)(int dtype, int head_dim, const Params& p, int row_waves, bool causal,
+                            unsigned grid, hipStream_t s, int variant);
 
 // One call's arguments, as the C ABI takes them.
 struct LaunchArgs {
@@ -422,6 +505,8 @@ struct LaunchArgs {
   bool static_order;
   // false: the launch may use its stream's ticket set but not make one (fa2_attn_fwd_noalloc)
   bool new_ticket_set = true;
+  // the general kernel whatever the shape (the measurement library's map of its program order)
+  bool general_only = false;
 };
 
 // A checked call, ready to launch: the kernel's arguments (without the key-norm table and the
@@ -431,6 +516,7 @@ struct LaunchPlan {
   int di = 0, waves = 1, bn = 64, splits = 1;
   int64_t grid = 0;         // workgroups, the dynamic tail's included
   bool empty = false;       // nothing to launch (an empty output)
+  int row_waves = 0;        // > 0: the wave-split kernel, 32 * row_waves rows a workgroup
   bool key_table = false;   // run the key-norm pass into key_table_at
   size_t key_table_at = 0;  // its byte offset in the workspace
   TailSchedule tail;        // tail_wgs == 0: the static order
@@ -554,33 +640,72 @@ int plan_launch(const LaunchArgs& a, const Topology& topo, LaunchPlan* out,
   p.static_blocks = 0x7fffffff;
   p.tail_queues = 1;
 
-  // Split-KV: cut the key range into whole tiles; drop splits that would be empty.
-  const int64_t kv_tiles = ((int64_t)a.n_kv + bn - 1) / bn;
+  // Key-norm table: used whenever the workspace has room for it beyond the split-KV partials of
+  // the REQUESTED split count, fa2_workspace_bytes(..., num_splits), which is where
+  // fa2_workspace_bytes_for puts it where it pays. The partials of a clamped (smaller) split
+  // count fit inside that size, so the room they leave never turns the table on by itself.
+  const size_t split_bytes =
+      a.num_splits > 1 ? workspace_layout((size_t)p.part_rows, a.head_dim, a.num_splits).total : 0;
+  const size_t table_bytes = key_table_bytes(a.batch, a.h_kv, a.n_kv);
+  const bool table_room = a.workspace && a.n_kv > 0 &&
+                          a.workspace_bytes >= split_bytes + table_bytes && a.variant == 0 &&
+                          waves == 4 && bn == default_block_n(a.head_dim);
+
+  // The kernel: the general one, or the wave-split one, whose rows are a KV head's whole group
+  // whatever pack. A caller that brings the table's room asks for the instance that uses it.
+  int kv_bn = bn;
   int splits = a.num_splits;
-  if (splits > 1 && kv_tiles > 0) {
-    const int64_t per = (kv_tiles + splits - 1) / splits;
-    splits = (int)((kv_tiles + per - 1) / per);
-    p.split_tiles = (int32_t)per;
+  if (!table_room && !a.general_only &&
+      (a.variant == 0 || a.variant == fa2::kVariantMaskEveryTile)) {
+    const KernelChoice kc =
+        kernel_choice(a.batch, a.h_q, a.h_kv, a.n_q, a.n_kv, a.head_dim, a.causal != 0, a.block_m,
+                      bn, topo.cus, a.num_splits);
+    if (kc.row_waves) {
+      pl.row_waves = kc.row_waves;
+      splits = kc.splits;
+      kv_bn = fa2::wave_split_block_n(a.head_dim, kc.row_waves, a.causal != 0);
+      const int64_t tile_rows = 32 * kc.row_waves;
+      p.n_tiles = (int32_t)(((int64_t)a.n_q * group + tile_rows - 1) / tile_rows);
+      p.n_bh = (int32_t)((int64_t)a.batch * a.h_kv);
+    }
   }
-  if (splits <= 1 || a.n_kv == 0) splits = 1;
+
+  // Split-KV: cut the key range into whole tiles; drop splits that would be empty. The workspace
+  // must hold the partials of the requested count at the general kernel's tiles, whichever kernel
+  // runs and however few splits it takes.
+  auto clamp_splits = [](int64_t tiles, int n) {
+    const int64_t per = (tiles + n - 1) / n;
+    return (int)((tiles + per - 1) / per);
+  };
+  const int need =
+      a.num_splits > 1 && a.n_kv > 0 ? clamp_splits(((int64_t)a.n_kv + bn - 1) / bn, a.num_splits) : 1;
+  splits = std::min(splits, need);
   if (splits > 1) {
-    const WorkspaceLayout w = workspace_layout((size_t)p.part_rows, a.head_dim, splits);
+    const int64_t kv_tiles = ((int64_t)a.n_kv + kv_bn - 1) / kv_bn;
+    p.split_tiles = (int32_t)((kv_tiles + splits - 1) / splits);
+    splits = clamp_splits(kv_tiles, splits);
+  }
+  if (need > 1) {
+    const WorkspaceLayout w = workspace_layout((size_t)p.part_rows, a.head_dim, need);
     if (!a.workspace || a.workspace_bytes < w.total)
       return fail(FA2_EINVAL, "split-KV with %d splits needs a workspace of %zu bytes, got %zu",
-                  splits, w.total, a.workspace ? a.workspace_bytes : (size_t)0);
+                  need, w.total, a.workspace ? a.workspace_bytes : (size_t)0);
     if (reinterpret_cast<uintptr_t>(a.workspace) & 255u)
       return fail(FA2_EALIGN, "the workspace must be 256-byte aligned");
+    // the combine pass runs one thread per 4 dims of every row
+    if (p.part_rows * (a.head_dim / 4) / 256 >= 0x7fffffffLL)
+      return fail(FA2_EINVAL, "split-KV merge of %lld rows is too large", (long long)p.part_rows);
+  }
+  if (splits > 1) {
+    const WorkspaceLayout w = workspace_layout((size_t)p.part_rows, a.head_dim, splits);
     p.part_o = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + w.part_o);
     p.part_lse = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + w.part_lse);
     p.part_lse_exact = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + w.part_lse_exact);
     p.splits = splits;
-    // the combine pass runs one thread per 4 dims of every row
-    if (p.part_rows * (a.head_dim / 4) / 256 >= 0x7fffffffLL)
-      return fail(FA2_EINVAL, "split-KV merge of %lld rows is too large", (long long)p.part_rows);
   } else {
     p.split_tiles = 0;
   }
-  int64_t grid = n_tiles * n_bh * splits;
+  int64_t grid = (int64_t)p.n_tiles * p.n_bh * splits;
   if (grid > 0x7fffffffLL)
     return fail(FA2_EINVAL, "grid of %lld workgroups is too large", (long long)grid);
   if (a.timeline) {  // the measurement library's timeline variant: kTimelineWords per program
@@ -591,15 +716,7 @@ int plan_launch(const LaunchArgs& a, const Topology& topo, LaunchPlan* out,
     p.timeline = a.timeline;
   }
 
-  // Key-norm table: used whenever the workspace has room for it beyond the split-KV partials of
-  // the REQUESTED split count, fa2_workspace_bytes(..., num_splits), which is where
-  // fa2_workspace_bytes_for puts it where it pays. The partials of a clamped (smaller) split
-  // count fit inside that size, so the room they leave never turns the table on by itself.
-  const size_t split_bytes =
-      a.num_splits > 1 ? workspace_layout((size_t)p.part_rows, a.head_dim, a.num_splits).total : 0;
-  const size_t table_bytes = key_table_bytes(a.batch, a.h_kv, a.n_kv);
-  if (a.workspace && a.n_kv > 0 && a.workspace_bytes >= split_bytes + table_bytes &&
-      a.variant == 0 && waves == 4 && bn == default_block_n(a.head_dim)) {
+  if (table_room) {
     if (reinterpret_cast<uintptr_t>(a.workspace) & 255u)
       return fail(FA2_EALIGN, "the workspace must be 256-byte aligned");
     const int64_t kgrid = (int64_t)a.batch * a.h_kv * ((a.n_kv + fa2::kKeyChunk - 1) / fa2::kKeyChunk);
@@ -608,7 +725,7 @@ int plan_launch(const LaunchArgs& a, const Topology& topo, LaunchPlan* out,
     pl.key_table = true;
     pl.key_table_at = split_bytes;
   }
-  if (!a.static_order)
+  if (!a.static_order && !pl.row_waves)
     pl.tail = tail_schedule(a.causal != 0, splits, waves, n_bh / (group / a.pack), group / a.pack,
                             n_tiles, p.unit_chunk, a.head_dim, bn, topo, tail_private_pct);
   if (pl.tail.tail_wgs > 0) grid = (int64_t)pl.tail.static_blocks + pl.tail.tail_wgs;
@@ -638,7 +755,8 @@ void apply_tail(LaunchPlan& pl, uint32_t* words) {
 
 // One call: plan it on the stream's device, then the key-norm pass, the attention kernel and the
 // split-KV merge, asynchronously on `stream`.
-int attn_fwd_impl(const LaunchArgs& a, KernelLaunch launch_kernel, void* stream) {
+int attn_fwd_impl(const LaunchArgs& a, KernelLaunch launch_kernel, SplitLaunch launch_split,
+                  void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int dev = stream_device(st);
   LaunchPlan pl;
@@ -675,8 +793,10 @@ int attn_fwd_impl(const LaunchArgs& a, KernelLaunch launch_kernel, void* stream)
   // marker of its own behind each launch (hipEventRecord) cost 0.6-1.8% (C3, C2, fp16 head_dim
   // 64), the event on the launch nothing measurable (same-box A/B)
   hipEvent_t stop = (set && FA2_TAIL_EVENT_GUARD) ? set->last : nullptr;
-  int e = launch_kernel(a.dtype, pl.di, p, pl.waves, pl.bn, a.causal != 0, (unsigned)grid, st,
-                        a.variant, stop);
+  int e = pl.row_waves ? launch_split(a.dtype, a.head_dim, p, pl.row_waves, a.causal != 0,
+                                      (unsigned)grid, st, a.variant)
+                        : launch_kernel(a.dtype, pl.di, p, pl.waves, pl.bn, a.causal != 0,
+                                        (unsigned)grid, st, a.variant, stop);
   if (set) {
     finish_tickets(set, e == hipSuccess);
     if (e == hipSuccess) g_tail_launches.fetch_add(1, std::memory_order_relaxed);

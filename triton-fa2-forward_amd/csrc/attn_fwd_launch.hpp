@@ -40,6 +40,22 @@ constexpr int default_block_n(int head_dim) { return head_dim == 16 ? 128 : 64; 
 // Launches the split-KV combine pass (attn_fwd_combine.hip).
 int launch_combine(int dtype, int head_dim, const CombineParams& c, hipStream_t stream);
 
+// The wave-split kernel (attn_fwd_wavesplit.hpp): keys per K/V tile of a key group, for 32
+// (row_waves 1) or 64 (2) rows per workgroup.
+constexpr int wave_split_block_n(int head_dim, int row_waves, bool causal) {
+  return head_dim == 128 ? 32 : head_dim == 64 || row_waves == 2 || causal ? 64 : 128;
+}
+// Launches it on `grid` workgroups of 32 * row_waves rows (p.n_tiles per KV head) and one split
+// each; p.split_tiles counts its tiles. VARIANT 0, or (measurement library) kVariantMaskEveryTile.
+template <int VARIANT>
+int launch_wave_split(int dtype, int head_dim, const Params& p, int row_waves, bool causal,
+                      unsigned grid, hipStream_t stream);
+template <>
+int launch_wave_split<0>(int, int, const Params&, int, bool, unsigned, hipStream_t);
+template <>
+int launch_wave_split<2 /* kVariantMaskEveryTile */>(int, int, const Params&, int, bool, unsigned,
+                                                     hipStream_t);
+
 // Launches the key-norm pass (attn_key_norm.hip) on `grid` = batch * h_kv * chunks workgroups.
 int launch_key_norm(int dtype, int head_dim, const KeyNormParams& k, unsigned grid,
                     hipStream_t stream);

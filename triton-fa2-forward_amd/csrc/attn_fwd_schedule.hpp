@@ -124,6 +124,53 @@ FA2_HD Program program_of(const Params& p, int block) {
   return pr;
 }
 
+// The wave-split kernel's programs (attn_fwd_wavesplit.hpp): n_tiles row tiles per (batch, KV head)
+// unit and `splits` key ranges each. As above, block b runs on XCD b % xcds.
+//   * Full: each XCD takes a contiguous run of the programs, unit after unit, so that a unit's row
+//     tiles share its K/V in one L2.
+//   * Causal: when the units split evenly over the XCDs each XCD owns whole units, else the row
+//     tiles of all units are dealt round-robin. Row tiles go heaviest first, every other round of
+//     one workgroup per CU in reverse, so that a CU's workgroups are a heavy and a light one (all
+//     of them are resident at once: the host takes the kernel for such grids only).
+struct SplitProgram {
+  int tile, split, b, hkv;
+};
+
+template <bool CAUSAL>
+FA2_HD SplitProgram split_program(const Params& p, int block) {
+  const int h_kv = p.h_q / p.group;
+  const int units = p.n_bh;  // batch * h_kv
+  const int xcds = 1 << p.xcd_shift;
+  SplitProgram pr;
+  int u;
+  if (CAUSAL) {
+    const bool local = (units & (xcds - 1)) == 0;
+    const int first = local ? (block & (xcds - 1)) * (units >> p.xcd_shift) : 0;  // XCD's first unit
+    const int own = local ? units >> p.xcd_shift : units;
+    const int round = local ? p.cus >> p.xcd_shift : p.cus;  // workgroups of one round
+    int slot = local ? block >> p.xcd_shift : block;
+    const int k = slot / round;
+    if (k & 1) slot = k * round + sched_min(round, own * p.n_tiles - k * round) - 1 - (slot - k * round);
+    const int t = slot / own;
+    u = first + slot - t * own;
+    pr.tile = p.n_tiles - 1 - t;
+    pr.split = 0;
+  } else {
+    const int per_u = p.n_tiles * p.splits;
+    const int total = units * per_u;
+    const int xcd = block & (xcds - 1);
+    const int i = xcd * (total >> p.xcd_shift) + sched_min(xcd, total & (xcds - 1)) +
+                  (block >> p.xcd_shift);
+    u = i / per_u;
+    const int r = i - u * per_u;
+    pr.split = r / p.n_tiles;
+    pr.tile = r - pr.split * p.n_tiles;
+  }
+  pr.b = u / h_kv;
+  pr.hkv = u - pr.b * h_kv;
+  return pr;
+}
+
 // ---- the dynamic tail's ticket -> program rules (Params: static_blocks .. tail_shared)
 
 // The queue of tail workgroup `block` (>= static_blocks): its XCD, as static_blocks is a

@@ -129,7 +129,7 @@ def build_variant(name, defines, jobs=8, verbose=False):
             cmds.append([cc, *flags, f"-DFA2_DT={dt}", f"-DFA2_D={d}", "-c",
                          os.path.join(CSRC, "attn_fwd_inst.hip"), "-o",
                          os.path.join(obj_dir, f"attn_fwd_dt{dt}_d{d}.o")])
-    for name_ in ("attn_fwd_combine", "attn_key_norm", "fa2_fwd", "fa2_scratch"):
+    for name_ in ("attn_fwd_combine", "attn_fwd_wavesplit", "attn_key_norm", "fa2_fwd", "fa2_scratch"):
         cmds.append([cc, *flags, "-c", os.path.join(CSRC, name_ + ".hip"), "-o",
                      os.path.join(obj_dir, name_ + ".o")])
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
@@ -158,7 +158,7 @@ def build(jobs=8, verbose=False):
             ablate_units.append([cc, *common_flags(), f"-DFA2_DT={dt}", f"-DFA2_D={d}", "-c",
                                  os.path.join(CSRC, "attn_fwd_ablate_inst.hip"), "-o", obj])
     shared = []
-    for name in ("attn_fwd_combine", "attn_key_norm"):
+    for name in ("attn_fwd_combine", "attn_fwd_wavesplit", "attn_key_norm"):
         shared.append([cc, *common_flags(), "-c", os.path.join(CSRC, name + ".hip"),
                        "-o", os.path.join(OBJ_DIR, name + ".o")])
     api = [cc, *common_flags(), "-c", os.path.join(CSRC, "fa2_fwd.hip"),
@@ -167,9 +167,12 @@ def build(jobs=8, verbose=False):
                "-o", os.path.join(OBJ_DIR, "fa2_scratch.o")]
     ablate_api = [cc, *common_flags(), "-c", os.path.join(CSRC, "fa2_ablate.hip"),
                   "-o", os.path.join(OBJ_DIR, "fa2_ablate.o")]
+    ablate_split = [cc, *common_flags(), "-DFA2_WAVE_SPLIT_VARIANT=2", "-c",
+                    os.path.join(CSRC, "attn_fwd_wavesplit.hip"),
+                    "-o", os.path.join(OBJ_DIR, "attn_fwd_wavesplit_ablate.o")]
     ceiling = [cc, *common_flags(), "-c", os.path.join(CSRC, "mfma_ceiling.hip"),
                "-o", os.path.join(OBJ_DIR, "mfma_ceiling.o")]
-    everything = units + shared + [api, scratch] + ablate_units + [ablate_api, ceiling]
+    everything = units + shared + [api, scratch] + ablate_units + [ablate_api, ablate_split, ceiling]
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
         errs = list(ex.map(lambda cmd: _run(cmd, verbose), everything))
 
@@ -188,7 +191,7 @@ def build(jobs=8, verbose=False):
 
     shared_objs = [u[-1] for u in shared]
     link([u[-1] for u in units] + shared_objs + [api[-1], scratch[-1]], LIB_PATH)
-    link([u[-1] for u in ablate_units] + shared_objs + [ablate_api[-1], ceiling[-1]],
+    link([u[-1] for u in ablate_units] + shared_objs + [ablate_api[-1], ablate_split[-1], ceiling[-1]],
          ABLATE_LIB_PATH)
     build_capi_check(verbose)
     return LIB_PATH

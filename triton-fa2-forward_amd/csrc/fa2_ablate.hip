@@ -28,11 +28,21 @@ int launch_ablate(int dtype, int di, const Params& p, int waves, int block_n, bo
   }
 }
 
+// The wave-split kernel has one timing variant, the one that must equal the product bit for bit.
+int launch_split_ablate(int dtype, int head_dim, const Params& p, int row_waves, bool causal,
+                        unsigned grid, hipStream_t s, int variant) {
+  if (variant == 0) return fa2::launch_wave_split<0>(dtype, head_dim, p, row_waves, causal, grid, s);
+  if (variant != fa2::kVariantMaskEveryTile) return (int)hipErrorInvalidValue;
+  return fa2::launch_wave_split<fa2::kVariantMaskEveryTile>(dtype, head_dim, p, row_waves, causal,
+                                                            grid, s);
+}
+
 // The plan of a launch of contiguous [B, H, N, D] tensors at block_m rows and the default
 // tile, without a workspace (no split-KV, no key-norm table), on `topo`. No device call.
 int plan_default(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, int32_t head_dim,
                  int32_t causal, int32_t pack, int32_t block_m, const Topology& topo,
-                 bool static_order, LaunchPlan* pl, int private_pct = FA2_TAIL_PRIVATE_PCT) {
+                 bool static_order, LaunchPlan* pl, int private_pct = FA2_TAIL_PRIVATE_PCT,
+                 bool general_only = true) {
   if (batch < 1 || h_q < 1 || h_kv < 1 || n_q < 1 || h_q % h_kv)
     return fail(FA2_EINVAL, "bad sizes: batch=%d h_q=%d h_kv=%d n_q=%d", batch, h_q, h_kv, n_q);
   const int64_t d = head_dim;
@@ -40,9 +50,10 @@ int plan_default(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, int32_t 
   const int64_t sk[4] = {(int64_t)h_kv * n_q * d, (int64_t)n_q * d, d, 1};
   // stand-in device addresses: the plan checks their alignment and never dereferences them
   void* const fake = reinterpret_cast<void*>(uintptr_t(1) << 20);
-  const LaunchArgs a{fake, fake, fake, fake, sq, sk, sk, sq, batch, h_q, h_kv, n_q, n_q,
-                     head_dim, FA2_DTYPE_BF16, causal, pack, block_m, 0, 1.0f, nullptr, 1,
-                     nullptr, 0, 0, nullptr, 0, static_order};
+  LaunchArgs a{fake, fake, fake, fake, sq, sk, sk, sq, batch, h_q, h_kv, n_q, n_q,
+               head_dim, FA2_DTYPE_BF16, causal, pack, block_m, 0, 1.0f, nullptr, 1,
+               nullptr, 0, 0, nullptr, 0, static_order};
+  a.general_only = general_only;
   return plan_launch(a, topo, pl, private_pct);
 }
 
@@ -76,7 +87,7 @@ int fa2_ablate_attn_fwd(const void* q, const void* k, const void* v, void* out,
   const LaunchArgs a{q, k, v, out, q_stride, k_stride, v_stride, o_stride, batch, h_q, h_kv,
                      n_q, n_kv, head_dim, dtype, causal, pack, 128, 0, qk_scale, nullptr, 1,
                      nullptr, 0, variant, nullptr, 0, static_order};
-  return attn_fwd_impl(a, launch_ablate, stream);
+  return attn_fwd_impl(a, launch_ablate, launch_split_ablate, stream);
 }
 
 int fa2_ablate_timeline(const void* q, const void* k, const void* v, void* out,
@@ -92,7 +103,7 @@ int fa2_ablate_timeline(const void* q, const void* k, const void* v, void* out,
   const LaunchArgs a{q, k, v, out, q_stride, k_stride, v_stride, o_stride, batch, h_q, h_kv,
                      n_q, n_kv, head_dim, dtype, causal, pack, 128, 0, qk_scale, nullptr, 1,
                      nullptr, 0, fa2::kVariantTimeline, records, record_words, false};
-  return attn_fwd_impl(a, launch_ablate, stream);
+  return attn_fwd_impl(a, launch_ablate, launch_split_ablate, stream);
 }
 
 int fa2_ablate_tail_schedule(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q,
@@ -126,7 +137,8 @@ int fa2_ablate_program_map(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q
   LaunchPlan pl;
   const int rc = plan_default(batch, h_q, h_kv, n_q, head_dim, causal, pack, block_m,
                               make_topology(cus, xcds), static_order != 0, &pl,
-                              tail_private_pct < 0 ? FA2_TAIL_PRIVATE_PCT : tail_private_pct);
+                              tail_private_pct < 0 ? FA2_TAIL_PRIVATE_PCT : tail_private_pct,
+                              static_order != 2);
   if (rc != FA2_OK) return rc;
   const int64_t grid = pl.empty ? 0 : pl.grid;
   if (program_words < 3 * grid)
@@ -161,7 +173,18 @@ int fa2_ablate_program_map(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q
     o[1] = pr.b;
     o[2] = pr.hq0;
   };
-  for (int64_t w = 0; w < first_tail; ++w) put(w, (int)w);
+  if (pl.row_waves) {  // static_order 2: the wave-split kernel's order
+    for (int64_t w = 0; w < grid; ++w) {
+      const fa2::SplitProgram pr = causal ? fa2::split_program<true>(p, (int)w)
+                                          : fa2::split_program<false>(p, (int)w);
+      int32_t* o = programs + 3 * w;
+      o[0] = pr.tile;
+      o[1] = pr.b;
+      o[2] = pr.hkv * p.group;
+    }
+    p.unit_chunk = 32 * pl.row_waves;
+  } else
+    for (int64_t w = 0; w < first_tail; ++w) put(w, (int)w);
   for (int32_t w : order) put(w, fa2::tail_pick(p, w, inc));
   int nonzero = 0;
   for (uint32_t x : words) nonzero += x != 0;

@@ -28,6 +28,12 @@ int launch(int dtype, int di, const Params& p, int waves, int block_n, bool caus
   }
 }
 
+int launch_split(int dtype, int head_dim, const Params& p, int row_waves, bool causal,
+                 unsigned grid, hipStream_t s, int variant) {
+  if (variant != 0) return (int)hipErrorInvalidValue;
+  return fa2::launch_wave_split<0>(dtype, head_dim, p, row_waves, causal, grid, s);
+}
+
 }  // namespace
 
 extern "C" {
@@ -105,9 +111,13 @@ int32_t fa2_num_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, in
   // Split until every CU has a workgroup, with at least kMinSplitTiles tiles per split and at
   // most kMaxSplits splits. (Filling the second workgroup slot of each CU as well measured
   // slower on MI355X: the fp32 partial outputs cost more than the extra overlap gains.)
+  // (The wave-split kernel's few-rows launches have a count of their own, which can be larger; where
+  // it is smaller the launch itself takes fewer than it is given.)
   int s = 1;
   while (programs * s < num_cus && s * 2 <= kMaxSplits && tiles / (s * 2) >= kMinSplitTiles) s *= 2;
-  return s;
+  const KernelChoice kc = kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, false, block_m, bn,
+                                        num_cus, kMaxSplits);
+  return kc.row_waves ? std::max(s, kc.splits) : s;
 }
 
 int fa2_attn_fwd_ex(const void* q, const void* k, const void* v, void* out,
@@ -120,7 +130,7 @@ int fa2_attn_fwd_ex(const void* q, const void* k, const void* v, void* out,
   const LaunchArgs a{q, k, v, out, q_stride, k_stride, v_stride, o_stride, batch, h_q, h_kv,
                      n_q, n_kv, head_dim, dtype, causal, pack, block_m, block_n, qk_scale, lse,
                      num_splits, workspace, workspace_bytes, 0, nullptr, 0, false};
-  return attn_fwd_impl(a, launch, stream);
+  return attn_fwd_impl(a, launch, launch_split, stream);
 }
 
 }  // extern "C"
@@ -176,7 +186,7 @@ int fa2_attn_fwd_noalloc(const void* q, const void* k, const void* v, void* out,
   const LaunchArgs a{q, k, v, out, q_stride, k_stride, v_stride, o_stride, batch, h_q, h_kv,
                      n_q, n_kv, head_dim, dtype, causal, pack, block_m, block_n, qk_scale, lse,
                      num_splits, ws, use, 0, nullptr, 0, false, false};
-  return attn_fwd_impl(a, launch, stream);
+  return attn_fwd_impl(a, launch, launch_split, stream);
 }
 
 }  // extern "C"

@@ -98,8 +98,10 @@ def attention(q, k, v, causal=True, sm_scale=None, block_m=None, block_n=None,
     Keyword-only extensions (the reference has neither, README.md:308-315):
     num_splits: split-KV, cut every program's key range into this many workgroups and merge
         their partial results in a second kernel (non-causal only); None picks it from the
-        grid size and the GPU's CU count (1 when the grid already fills the GPU). The pick
-        does not depend on pack_gqa, so packed and unpacked results stay equal bit for bit.
+        grid size and the GPU's CU count (1 when the grid already fills the GPU). At the default
+        tiles, few rows per KV head and small grids share a row's keys among a workgroup's waves
+        first and take at most this many splits. The pick does not depend on pack_gqa, so packed
+        and unpacked results stay equal bit for bit.
     return_lse: also return the natural-log log-sum-exp of every row's scaled scores, fp32
         [B, H_q, N_q], i.e. (out, lse).
     """
