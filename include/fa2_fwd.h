@@ -192,6 +192,16 @@ FA2_API int32_t fa2_num_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t
                                int32_t num_cus);
 
 /*
+ * fa2_launch_splits - the split count that a launch given num_splits takes: fewer where the kernel
+ * for few rows and small grids (see fa2_attn_fwd_ex) needs fewer, else num_splits. A caller that
+ * passes this count gets the same output, bit for bit, and needs the workspace of this count only
+ * (none for 1). block_n 0 takes the default. Host policy only.
+ */
+FA2_API int32_t fa2_launch_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, int32_t n_kv,
+                                  int32_t head_dim, int32_t causal, int32_t block_m, int32_t block_n,
+                                  int32_t num_cus, int32_t num_splits);
+
+/*
  * fa2_default_config - the gfx950 tile configuration for a head dim.
  * Replaces `_default_config(head_dim, on_cuda)` (fa2/kernel.py:186-195). Writes
  * block_m (rows per program), block_n (keys per K/V tile), num_waves (wave64s per

@@ -6,7 +6,8 @@ measurement library libfa2_ablate.so beside it.
 Compiles attn_fwd_inst.hip once per (dtype, head_dim) pair plus the split-KV combine pass
 (attn_fwd_combine.hip), the key-norm pass (attn_key_norm.hip) and the C-ABI file fa2_fwd.hip,
 in parallel, with hipcc for gfx950 only, and links them into
-triton-fa2-forward_amd/fa2/libfa2_fwd.so next to the Python front end that loads it. Then builds
+triton-fa2-forward_amd/fa2/libfa2_fwd.so next to the Python front end that loads it. Beside it goes
+fa2/_torch_call.so, the front end's native common call (fa2_torch.cpp, against the installed torch). Then builds
 the plain-C host of the C ABI that the tests run (tests/capi/fa2_capi_check).
 
 The measurement library (include/fa2_ablate.h) is the kernel's timing variants: the same kernel
@@ -41,6 +42,7 @@ ROOT = os.path.dirname(PKG)
 INCLUDE = os.path.join(ROOT, "include")
 OBJ_DIR = os.path.join(PKG, "build", "obj")
 LIB_PATH = os.path.join(PKG, "fa2", "libfa2_fwd.so")
+TORCH_CALL_PATH = os.path.join(PKG, "fa2", "_torch_call.so")
 ABLATE_LIB_PATH = os.path.join(PKG, "libfa2_ablate.so")
 RESOURCES_PATH = os.path.join(PKG, "fa2", "kernel_resources.json")
 CAPI_DIR = os.path.join(ROOT, "tests", "capi")
@@ -172,7 +174,12 @@ def build(jobs=8, verbose=False):
                     "-o", os.path.join(OBJ_DIR, "attn_fwd_wavesplit_ablate.o")]
     ceiling = [cc, *common_flags(), "-c", os.path.join(CSRC, "mfma_ceiling.hip"),
                "-o", os.path.join(OBJ_DIR, "mfma_ceiling.o")]
-    everything = units + shared + [api, scratch] + ablate_units + [ablate_api, ablate_split, ceiling]
+    torch_obj = os.path.join(OBJ_DIR, "fa2_torch.o")
+    torch_call = ["g++", "-std=c++20", "-O2", "-fPIC", "-fvisibility=hidden", "-Wall",
+                  "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", "-I", INCLUDE,
+                  *(f for p in torch_paths()[0] for f in ("-isystem", p)), "-c",
+                  os.path.join(CSRC, "fa2_torch.cpp"), "-o", torch_obj]
+    everything = units + shared + [api, scratch] + ablate_units + [ablate_api, ablate_split, ceiling, torch_call]
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
         errs = list(ex.map(lambda cmd: _run(cmd, verbose), everything))
 
@@ -193,8 +200,27 @@ def build(jobs=8, verbose=False):
     link([u[-1] for u in units] + shared_objs + [api[-1], scratch[-1]], LIB_PATH)
     link([u[-1] for u in ablate_units] + shared_objs + [ablate_api[-1], ablate_split[-1], ceiling[-1]],
          ABLATE_LIB_PATH)
+    _run(["g++", "-shared", "-fPIC", "-o", TORCH_CALL_PATH + ".tmp", torch_obj,
+          "-L", os.path.dirname(LIB_PATH), "-lfa2_fwd", "-L", torch_paths()[1], "-ltorch_python",
+          "-ltorch_cpu", "-ltorch", "-lc10_hip", "-lc10",
+          "-L", os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hipcc()))), "lib"),
+          "-lamdhip64", "-Wl,-rpath,$ORIGIN"], verbose)
+    os.replace(TORCH_CALL_PATH + ".tmp", TORCH_CALL_PATH)
     build_capi_check(verbose)
     return LIB_PATH
+
+
+def torch_paths():
+    """(include directories, library directory) of this interpreter's torch and Python."""
+    import importlib.util
+    import sysconfig
+
+    torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    inc = os.path.join(torch_dir, "include")
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
+    return ([inc, os.path.join(inc, "torch", "csrc", "api", "include"),
+             sysconfig.get_paths()["include"], os.path.join(rocm, "include")],
+            os.path.join(torch_dir, "lib"))
 
 
 def build_capi_check(verbose=False):

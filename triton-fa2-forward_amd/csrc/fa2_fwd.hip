@@ -120,6 +120,16 @@ int32_t fa2_num_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, in
   return kc.row_waves ? std::max(s, kc.splits) : s;
 }
 
+int32_t fa2_launch_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, int32_t n_kv,
+                          int32_t head_dim, int32_t causal, int32_t block_m, int32_t block_n,
+                          int32_t num_cus, int32_t num_splits) {
+  if (num_splits <= 1 || causal || batch <= 0 || h_q <= 0 || h_kv <= 0 || h_q % h_kv || n_q <= 0 ||
+      n_kv <= 0 || block_m <= 0 || num_cus <= 0 || dim_index(head_dim) < 0)
+    return num_splits;
+  return kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, false, block_m,
+                       tile_n(block_n, head_dim), num_cus, num_splits).splits;
+}
+
 int fa2_attn_fwd_ex(const void* q, const void* k, const void* v, void* out,
                     const int64_t q_stride[4], const int64_t k_stride[4],
                     const int64_t v_stride[4], const int64_t o_stride[4],

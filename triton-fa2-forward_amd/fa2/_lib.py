@@ -30,6 +30,7 @@ SIGNATURES = {
     "fa2_workspace_bytes_for": (ctypes.c_size_t, [_i32, _i32, _i32, _i32, _i32, _i32, _i32,
                                                   _i32, _i32]),
     "fa2_num_splits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
+    "fa2_launch_splits": (_i32, [_i32] * 11),
     "fa2_default_config": (ctypes.c_int, [_i32, ctypes.POINTER(_i32), ctypes.POINTER(_i32),
                                           ctypes.POINTER(_i32), ctypes.POINTER(_i32)]),
     "fa2_should_pack_gqa": (ctypes.c_int, [_i32, _i32, _i32]),
@@ -57,6 +58,15 @@ def lib():
             fn.argtypes = argtypes
         _LIB = handle
     return _LIB
+
+
+# The native common call of attention() (csrc/fa2_torch.cpp), built beside the library against this
+# torch; None where it is missing or was built for another torch: attention() then makes every
+# call itself, through ctypes.
+try:
+    from ._torch_call import call as fast_call
+except ImportError:
+    fast_call = None
 
 
 def last_error():

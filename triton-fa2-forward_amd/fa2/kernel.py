@@ -105,6 +105,13 @@ def attention(q, k, v, causal=True, sm_scale=None, block_m=None, block_n=None,
     return_lse: also return the natural-log log-sum-exp of every row's scaled scores, fp32
         [B, H_q, N_q], i.e. (out, lse).
     """
+    # the common call, made natively; None: not one of those
+    if (block_m is block_n is num_warps is num_stages is pack_gqa is num_splits is None
+            and _lib.fast_call is not None):
+        result = _lib.fast_call(q, k, v, causal, sm_scale, return_lse)
+        if result is not None:
+            return result
+
     assert q.dim() == k.dim() == v.dim() == 4
     B, H_q, N_q, D = q.shape
     Bk, H_kv, N_kv, Dk = k.shape
