@@ -185,6 +185,24 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
   return kc;
 }
 
+// Whether a full (not causal) call at the default tiles runs the wide kernel (attn_fwd_wide.hpp),
+// whose programs of 256 rows a CU holds two of: bit for bit the same output as the general kernel's
+// 128-row programs. Measured on MI355X (general -> wide, us; `rounds` of two programs per CU), H16 D64
+// unless stated: one round B8 N1024 45.3 -> 44.7, B4 N2048 82.9 -> 79.5, B2 N4096 156.0 -> 149.7; 1.5
+// B12 N1024 68.2 -> 66.6, 1.76 B5 H12 N3840 265.4 -> 253.0; 2 B4 N4096 305.6 -> 292.7; 3 B12 N2048
+// 237.7 -> 227.3, D32 160.6 -> 151.9. A last round that only a few programs reach costs more than that:
+// 1.12 rounds B3 H12 N4096 180.4 -> 199.8, 1.25 B5 N2048 101.4 -> 109.7; 0.75 B6 N1024 36.0 -> 40.4. So
+// do rows past the last (N3186: 13 programs of 256 rows for 24.9 of 128) 582.1 -> 590.2, and short key
+// ranges (B16 N512 27.6 -> 27.9).
+bool wide_pays(int64_t rows, int64_t n_bh, int64_t n_kv, int32_t head_dim, int cus) {
+  if ((head_dim != 32 && head_dim != 64) || n_kv < 1024) return false;
+  const int64_t tiles = (rows + fa2::kWideRows - 1) / fa2::kWideRows;
+  if (tiles * 2 * 100 > (rows + 127) / 128 * 102) return false;
+  const int64_t programs = tiles * n_bh, round = 2 * (int64_t)cus;
+  const int64_t past = programs % round;  // programs of the last, partial round
+  return programs >= round && (past == 0 || 10 * past >= 4 * round || programs >= 3 * round);
+}
+
 // Topology of a device as the program order uses it: log2 of its XCD count and its CU count.
 struct Topology {
   int32_t xcd_shift = 3;  // 8 XCDs
@@ -507,6 +525,8 @@ struct LaunchArgs {
   bool new_ticket_set = true;
   // the general kernel whatever the shape (the measurement library's map of its program order)
   bool general_only = false;
+  // the library's own launches may take the wide kernel (the measurement library has no instance)
+  bool wide_ok = false;
 };
 
 // A checked call, ready to launch: the kernel's arguments (without the key-norm table and the
@@ -668,6 +688,12 @@ int plan_launch(const LaunchArgs& a, const Topology& topo, LaunchPlan* out,
       p.n_tiles = (int32_t)(((int64_t)a.n_q * group + tile_rows - 1) / tile_rows);
       p.n_bh = (int32_t)((int64_t)a.batch * a.h_kv);
     }
+  }
+
+  if (a.wide_ok && !pl.row_waves && a.num_splits == 1 && a.block_m == 128 && bn == 64 && !a.causal &&
+      wide_pays(rows, n_bh, a.n_kv, a.head_dim, topo.cus)) {
+    p.block_m = fa2::kWideRows;
+    p.n_tiles = (int32_t)((rows + fa2::kWideRows - 1) / fa2::kWideRows);
   }
 
   // Split-KV: cut the key range into whole tiles; drop splits that would be empty. The workspace

@@ -2,6 +2,7 @@
 // Compiled once per pair with -DFA2_DT=<0 fp16 | 1 bf16> -DFA2_D=<16|32|64|128>.
 #include "attn_fwd_kernel.hpp"
 #include "attn_fwd_launch.hpp"
+#include "attn_fwd_wide.hpp"
 
 #if !defined(FA2_DT) || !defined(FA2_D)
 #error "compile with -DFA2_DT=<0|1> -DFA2_D=<16|32|64|128>"
@@ -32,6 +33,14 @@ int launch_bn(const Params& p, int block_n, bool causal, unsigned grid, hipStrea
 template <int DT, int D>
 int launch_attn_fwd(const Params& p, int waves, int block_n, bool causal, unsigned grid,
                     hipStream_t s, hipEvent_t stop) {
+  if constexpr (D == 32 || D == 64) {
+    if (waves == 4 && p.block_m == kWideRows) {  // 64 rows a wave (attn_fwd_wide.hpp)
+      if (block_n != 64 || causal) return (int)hipErrorInvalidValue;
+      if (p.key_norm2)
+        return launch_with_stop(attn_wide_kernel<DT, D, true>, grid, 256, s, stop, p);
+      return launch_with_stop(attn_wide_kernel<DT, D, false>, grid, 256, s, stop, p);
+    }
+  }
   if (p.key_norm2) {  // the host writes a key-norm table only for the default configuration
     constexpr int BN = default_block_n(D);
     if (waves != 4 || block_n != BN) return (int)hipErrorInvalidValue;

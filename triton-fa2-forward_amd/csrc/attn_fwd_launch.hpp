@@ -31,6 +31,11 @@ template <int DT, int D>
 int launch_attn_fwd(const Params& p, int waves, int block_n, bool causal, unsigned grid,
                     hipStream_t stream, hipEvent_t stop);
 
+// Rows of a program of the wide kernel (attn_fwd_wide.hpp), which launch_attn_fwd runs for
+// waves 4 and p.block_m of this many rows (head_dim 32 and 64, not
+// causal, 64-key tiles, one split).
+constexpr int kWideRows = 256;
+
 // gfx950 default K/V tile: 64 keys (sweep.py on the BASELINE.json configs, MI355X: best for
 // C2, C3, C5 at head_dim 128, and for C4 at head_dim 64 with the software-pipelined loop that
 // 64-key tiles get there; a tie with 128 at head_dim 32); 128 keys at head_dim 16 (+2.4% causal,

@@ -139,7 +139,7 @@ int fa2_attn_fwd_ex(const void* q, const void* k, const void* v, void* out,
                     int32_t num_splits, void* workspace, size_t workspace_bytes, void* stream) {
   const LaunchArgs a{q, k, v, out, q_stride, k_stride, v_stride, o_stride, batch, h_q, h_kv,
                      n_q, n_kv, head_dim, dtype, causal, pack, block_m, block_n, qk_scale, lse,
-                     num_splits, workspace, workspace_bytes, 0, nullptr, 0, false};
+                     num_splits, workspace, workspace_bytes, 0, nullptr, 0, false, true, false, true};
   return attn_fwd_impl(a, launch, launch_split, stream);
 }
 
@@ -195,7 +195,7 @@ int fa2_attn_fwd_noalloc(const void* q, const void* k, const void* v, void* out,
   }
   const LaunchArgs a{q, k, v, out, q_stride, k_stride, v_stride, o_stride, batch, h_q, h_kv,
                      n_q, n_kv, head_dim, dtype, causal, pack, block_m, block_n, qk_scale, lse,
-                     num_splits, ws, use, 0, nullptr, 0, false, false};
+                     num_splits, ws, use, 0, nullptr, 0, false, false, false, true};
   return attn_fwd_impl(a, launch, launch_split, stream);
 }
 
