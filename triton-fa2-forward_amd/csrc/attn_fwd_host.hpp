@@ -118,7 +118,25 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
 //   * few rows (at most 64 per KV head, not causal), bound by reading K/V: bf16 H32/8 D128 one
 //     query of 32000 keys 50.5 -> 32.4, of 1000 10.1 -> 7.9, B16 4096 keys 59.9 -> 49.4, B16 with 16
 //     queries 62.2 -> 53.4, H28/4 D64 B8 5712 keys 53.4 -> 15.1 (the general kernel cannot pack a
-//     group of 7); B40 of 2000 keys 65.2 -> 67.8 is the one loss seen.
+//     group of 7).
+//   * few rows in more 32-row workgroups than CUs. 33 to 64 rows: two row tiles read every key twice,
+//     so 64 rows a workgroup, or, where the general kernel packs the group, its one program (general /
+//     32 / 64 rows a workgroup; units are KV heads): D128 336 units 64 rows 206 keys 12.8 / 16.0 / 13.7,
+//     2000 67.9 / 74.5 / 68.9; 160 units 48 rows 206 keys 9.0 / 10.3 / 8.7, 700 19.6 / 16.4 / 14.8, 4000
+//     (the general kernel splits) 70.4 / 83.5 / 81.2; 248 units 64 rows 700 keys 31.1 / 21.0 / 20.4. D64
+//     336 units 64 rows 1000 keys 24.1 / 21.2 / 19.7, 136 units 36 rows 206 keys 7.0 / 6.9 / 6.1, but 600
+//     units (one round of the general kernel) 700 keys 28.0 / 29.9 / 29.3. D32 336 units 64 rows 2000
+//     keys 32.6 / 22.4 / 21.2, but 248 units of 4000 keys 44.1 / 28.7 / 32.6. Up to 32 rows: a last round that few workgroups reach costs the 32-row
+//     kernel more: D128 264 units 4 rows 2000 keys 56.6 / 62.7 / 53.9, 448 units 80.6 / 78.5 / 79.5; 264
+//     units 32 rows 206 keys 10.7 / 11.2 / 11.2; D64 264 units 2000 keys 42.0 / 32.9 / 30.2, 1000 21.3 /
+//     15.4 / 15.9; D32 336 units 206 keys 7.1 / 6.3 / 5.9, 2000 32.3 / 18.5 / 20.2.
+//   * more rows in groups that do not divide 128: the general kernel runs a program per query head,
+//     mostly of empty rows when it has few queries; full, general -> this kernel: D128 H28/4 B4 16
+//     queries of 8192 keys 50.3 -> 20.9, B1 20 of 8192 20.1 -> 15.1, B20 30 of 6000 233 -> 112, H20/4 B40
+//     16 of 1000 50.0 -> 26.0; D64 H28/4 B4 16 of 8192 39.5 -> 14.4. With long keys on grids of more than
+//     half the CUs 64 rows a workgroup and splits beat 32: B8 40 of 8000 99.4 / 89.6 / 75.0, H20/4 B12 64
+//     of 20000 277 / 293 / 200. It takes 1.5 times the rows' own slots to be worth it (2.5 below 512
+//     keys): H28/4 B1 200 of 8000 (1.27) 39.9 -> 45.2, B30 60 of 300 (2.0) 23.3 -> 24.8.
 //   * causal, one round of workgroups (D128 H8/2): N 512 12.5 -> 8.5, 1024 20.8 -> 11.5, 2048
 //     37.5 -> 20.9, 4096 (w2 512) 69.7 -> 55.1; H32/8 N 256 8.9 -> 7.4, 512 13.0 -> 10.7, 1024
 //     (w2 512) 22.7 -> 20.3, but 2048 (w2 1024) 45.8 -> 50.5. D64 H16 N 256 7.7 -> 5.7, 1024 16.0
@@ -144,6 +162,7 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
   if (rows > (int64_t(1) << 22) || units > (int64_t(1) << 22)) return kc;  // (products below fit)
   const int64_t w1 = (rows + 31) / 32 * units, w2 = (rows + 63) / 64 * units;
   const bool small = head_dim <= 32;
+  const bool packs = 128 % (h_q / h_kv) == 0;  // the general kernel can pack the group
   // The splits of a launch of 32-row workgroups: doubled until one more doubling would pass one
   // workgroup per CU or leave a wave without a tile, where a wave has tiles enough for the merge
   // launch (~2 us) to pay: 7 of 32 keys x D128, or 14 where only one doubling fits. Measured (us at
@@ -168,7 +187,30 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
       kc.row_waves = 2;
   } else if (rows <= 64) {
     kc.row_waves = 1;
-    take_splits();
+    if (w1 <= cus) {
+      take_splits();
+      return kc;
+    }
+    // more 32-row workgroups than CUs (the first list above)
+    kc.splits = 1;
+    if (rows > 32) {
+      bool general;  // where it packs: its one 128-row program is as good or better
+      if (head_dim == 128)
+        general = w1 > 2 * cus || (n_kv < 256 ? rows > 48 : n_kv >= 1024 && 4 * w1 <= 7 * cus);
+      else
+        general = head_dim == 64 && w2 > 2 * cus && w2 <= 3 * cus;
+      kc.row_waves = general && packs ? 0 : small && w1 <= 2 * cus && n_kv >= 1536 ? 1 : 2;
+    } else if (head_dim == 128) {
+      if (packs && rows > 24 && n_kv < 600 && 4 * w1 <= 5 * cus)
+        kc.row_waves = 0;
+      else if (n_kv >= 384 && 5 * w1 <= 8 * cus)
+        kc.row_waves = 2;
+    } else if (head_dim == 64) {
+      if (n_kv >= 1280 && 2 * w1 <= 3 * cus) kc.row_waves = 2;
+    } else if (n_kv < 320 || (n_kv < 768 && w1 > 2 * cus)) {
+      kc.row_waves = 2;
+    }
+    if (!kc.row_waves) kc.splits = max_splits;
   } else if (n_kv <= (head_dim == 128 ? 2048 : 4096)) {
     if (w1 <= cus) {
       kc.row_waves = 1;
@@ -178,6 +220,27 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
       kc.row_waves = 10 * w2 >= 9 * cus ? 2 : 1;
       kc.splits = 1;
     } else if (small && w2 <= 2 * cus && n_kv >= 512) {
+      kc.row_waves = 2;
+      kc.splits = 1;
+    }
+  }
+  if (!causal && !kc.row_waves && !packs && rows > 64) {
+    // 64-row slots the general kernel fills, of one query head each, against the rows' own
+    const int64_t slots = (n_q + 127) / 128 * 2 * (h_q / h_kv) * units;
+    if (w1 <= 2 * cus) {
+      if (2 * slots >= 3 * w2) {
+        if (!small && n_kv >= 6144 && 2 * w1 > cus) {
+          kc.row_waves = 2;
+          kc.splits = 1;
+          const int64_t tiles = n_kv / (2 * fa2::wave_split_block_n(head_dim, 2, false));
+          while (kc.splits * 2 <= max_splits && w2 * kc.splits <= cus && tiles / kc.splits >= 8)
+            kc.splits *= 2;
+        } else {
+          kc.row_waves = 1;
+          take_splits();
+        }
+      }
+    } else if (2 * slots >= (n_kv >= 512 ? 3 : 5) * w2) {
       kc.row_waves = 2;
       kc.splits = 1;
     }
