@@ -56,12 +56,13 @@ def test_causal(dtype, D, B, h_q, h_kv, n):
 
 
 # one shape per branch of the rule where 32-row workgroups outnumber the CUs (33 to 64 rows, then fewer)
-# and where the group does not divide 128 (small grid, long keys with splits, large grid)
+# where the group does not divide 128 (small grid, long keys with splits, large grid), and two to three
+# 64-row workgroups per CU (which head_dim 16 and 32 take)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("D", [16, 32, 64, 128])
 @pytest.mark.parametrize("B,h_q,h_kv,n_q,n_kv", [
     (17, 8, 8, 40, 300), (33, 16, 8, 20, 1100), (33, 28, 4, 7, 700), (33, 8, 8, 1, 1601), (34, 8, 8, 30, 230),
-    (1, 28, 4, 10, 4300), (8, 28, 4, 40, 6200), (20, 28, 4, 30, 4200)])
+    (1, 28, 4, 10, 4300), (8, 28, 4, 40, 6200), (20, 28, 4, 30, 4200), (4, 8, 8, 1201, 520), (1, 20, 4, 2000, 4100)])
 def test_full_past_one_workgroup_per_cu(dtype, D, B, h_q, h_kv, n_q, n_kv):
     _check(*make_qkv(B, h_q, h_kv, n_q, n_kv, D, dtype), causal=False)
 

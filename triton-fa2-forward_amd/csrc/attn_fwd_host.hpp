@@ -141,11 +141,18 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
 //     37.5 -> 20.9, 4096 (w2 512) 69.7 -> 55.1; H32/8 N 256 8.9 -> 7.4, 512 13.0 -> 10.7, 1024
 //     (w2 512) 22.7 -> 20.3, but 2048 (w2 1024) 45.8 -> 50.5. D64 H16 N 256 7.7 -> 5.7, 1024 16.0
 //     -> 9.3, 2048 (w2 512) 28.4 -> 20.7; B4 1024 (w2 1024) 19.9 -> 23.1. D32 H16 B2 N 2048 (w2
-//     1024; its small tiles let a CU hold four workgroups) 24.0 -> 20.0, B4 (w2 2048) 34.3 -> 36.6.
+//     1024; its small tiles let a CU hold four workgroups) 24.0 -> 20.0, B4 (w2 2048) 34.3 -> 36.6;
+//     w2 1024 with shorter keys: D32 N 1024 14.0 -> 13.0, 512 9.1 -> 10.0; D16 N 4096 34.2 -> 29.3, 2048
+//     19.2 -> 17.2, 1024 11.1 -> 11.4 (w2 768, N 1000: 11.0 -> 10.1).
 //   * full, more rows: H16 D64 N 512 9.2 -> 6.3, 1024 (w2 256) 14.4 -> 11.3, 2048 (w2 512) 27.5 ->
 //     27.2; B2 H16 D64 333 x 1500 20.7 -> 14.0; H32/8 D128 64 x 2048 B4 23.4 -> 17.2. Every row
 //     tile reads its KV head's keys again, so past some thousand keys the general kernel and its
 //     split are better: H32/8 D128 128 x 4096 24.6 -> 26.3, D64 H16 256 x 8192 23.0 -> 29.8.
+//   * full at head_dim 16 and 32 on w2 of 2 to 3 workgroups per CU: the general kernel's 128-row
+//     programs leave CUs with one beside CUs with two, and 64 rows spread more evenly, at any key
+//     count: D32 H8 4160 x 512 10.4 -> 9.7, x 4090 58.6 -> 42.6, x 16000 217.7 -> 148.2, 6144 x 16000
+//     217.4 -> 160.3; D16 4160 x 700 12.7 -> 11.4, x 16000 169.4 -> 150.9. Past three, D32 H16 4096 x 1000
+//     18.5 -> 19.4, D16 15.7 -> 17.1; up to two, D32 H8 4000 x 4090 41.9 -> 33.9 but D16 N 2048 18.0 -> 18.8.
 //   * up to 128 keys (192 at head_dim 128, where tiles are small) there is little to share out:
 //     D128 H32/8 N 64 5.1 -> 6.5, N 128 6.7 -> 6.6, N 192 7.3 -> 7.3.
 struct KernelChoice {
@@ -183,7 +190,9 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
   if (causal) {  // (num_splits is 1)
     if (w1 <= cus || (w1 <= 2 * cus && n_kv >= 384))
       kc.row_waves = 1;
-    else if (w2 <= (small ? 4 : 2) * cus && n_kv >= (head_dim == 128 ? 512 : 0))
+    else if (w2 <= 2 * cus && n_kv >= (head_dim == 128 ? 512 : 0))
+      kc.row_waves = 2;
+    else if (small && w2 <= 4 * cus && n_kv >= (head_dim == 16 && w2 > 3 * cus ? 1536 : 768))
       kc.row_waves = 2;
   } else if (rows <= 64) {
     kc.row_waves = 1;
@@ -219,10 +228,14 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
       // two workgroups on some CUs: 64 rows a workgroup where that still reaches every CU
       kc.row_waves = 10 * w2 >= 9 * cus ? 2 : 1;
       kc.splits = 1;
-    } else if (small && w2 <= 2 * cus && n_kv >= 512) {
+    } else if (head_dim == 32 && w2 <= 2 * cus && n_kv >= 512) {
       kc.row_waves = 2;
       kc.splits = 1;
     }
+  }
+  if (!causal && small && n_kv >= 512 && w2 > 2 * cus && w2 <= 3 * cus) {
+    kc.row_waves = 2;
+    kc.splits = 1;
   }
   if (!causal && !kc.row_waves && !packs && rows > 64) {
     // 64-row slots the general kernel fills, of one query head each, against the rows' own
