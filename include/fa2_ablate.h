@@ -199,6 +199,24 @@ FA2_API int fa2_ablate_program_map(int32_t batch, int32_t h_q, int32_t h_kv, int
                                    int32_t tail_private_pct, uint32_t seed, int32_t* programs,
                                    int64_t program_words, int32_t* info, int32_t info_words);
 
+/* Words fa2_ablate_plan writes to info. */
+#define FA2_ABLATE_PLAN_INFO_WORDS 7
+
+/*
+ * fa2_ablate_plan - what fa2_attn_fwd_ex launches for contiguous tensors of these sizes, given
+ * num_splits and a workspace of workspace_bytes (0: none), on a device of `cus` CUs and `xcds` XCDs:
+ * the library's own planning code, without a GPU call. Its errors are fa2_attn_fwd_ex's.
+ *   info      [FA2_ABLATE_PLAN_INFO_WORDS]: the kernel (0 general, 1 wave-split, 2 wide), rows per
+ *             workgroup, keys per K/V tile, key ranges (splits), K/V tiles per range (0 without
+ *             splits), workgroups, and 1 if the key-norm table is used.
+ * No counterpart in the reference: how tests and tools know which kernel a call runs.
+ */
+FA2_API int fa2_ablate_plan(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, int32_t n_kv,
+                            int32_t head_dim, int32_t dtype, int32_t causal, int32_t pack,
+                            int32_t block_m, int32_t block_n, int32_t num_splits,
+                            size_t workspace_bytes, int32_t cus, int32_t xcds, int32_t* info,
+                            int32_t info_words);
+
 /*
  * fa2_ablate_tail_launches - how many launches of this library (fa2_ablate_attn_fwd,
  * fa2_ablate_timeline) ran with a dynamic tail so far in this process: a launch recorded under

@@ -192,10 +192,14 @@ FA2_API int32_t fa2_num_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t
                                int32_t num_cus);
 
 /*
- * fa2_launch_splits - the split count that a launch given num_splits takes: fewer where the kernel
- * for few rows and small grids (see fa2_attn_fwd_ex) needs fewer, else num_splits. A caller that
- * passes this count gets the same output, bit for bit, and needs the workspace of this count only
- * (none for 1). block_n 0 takes the default. Host policy only.
+ * fa2_launch_splits - the number of key ranges that a launch given num_splits runs: at most that
+ * many, of whole K/V tiles and none empty, and fewer where the kernel for few rows and small
+ * grids (see fa2_attn_fwd_ex) needs fewer. A caller that passes this count instead makes the same
+ * ranges, gets the same output bit for bit, and needs the workspace of this count only (none for 1).
+ * Both launches' workspaces are of fa2_workspace_bytes: with room for the key-norm table beyond it
+ * (what fa2_workspace_bytes_for adds where the table pays) the kernel that uses the table runs
+ * instead, on every range asked for, so such a caller passes num_splits itself. block_n 0 takes the
+ * default. Host policy only.
  */
 FA2_API int32_t fa2_launch_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, int32_t n_kv,
                                   int32_t head_dim, int32_t causal, int32_t block_m, int32_t block_n,

@@ -410,7 +410,7 @@ def test_measurement_library_exports_exactly_its_header():
     assert {n for n in names if n.startswith("fa2_")} == _c_names(ABLATE_HEADER) == {
         "fa2_ablate_attn_fwd", "fa2_ablate_timeline", "fa2_ablate_mfma_ceiling",
         "fa2_ablate_hbm_read", "fa2_ablate_tail_schedule", "fa2_ablate_program_map",
-        "fa2_ablate_tail_launches", "fa2_ablate_last_error"}
+        "fa2_ablate_plan", "fa2_ablate_tail_launches", "fa2_ablate_last_error"}
     # the knockouts are compiled into it: kernel instances with the no_exp, no_softmax and
     # kv_l2 bits, matmul_only (no_softmax | kv_l2), no_kv_staging (256), the key split (512,
     # head_dim 128 only), no_q_load (1024) and no_store (2048); and the timeline instance (64)

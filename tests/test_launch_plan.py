@@ -1,0 +1,99 @@
+"""The split counts the library tells against the ones it runs, on the CPU: fa2_launch_splits and
+fa2_num_splits (include/fa2_fwd.h) against the plan of the launch itself (fa2_ablate_plan: the
+library's planning code, without a GPU call).
+"""
+
+import random
+
+import pytest
+
+from fa2 import _lib
+from test_schedule import needs_ablate
+
+WAVE_SPLIT = "fa2::attn_wave_split_kernel"
+
+
+def _plan(*sizes, **kw):
+    from ablation import launch_plan
+    return launch_plan(*sizes, **kw)
+
+
+def _launch_splits(B, h_q, h_kv, n_q, n_kv, D, num_splits, cus=256):
+    return int(_lib.lib().fa2_launch_splits(B, h_q, h_kv, n_q, n_kv, D, 0, 128, 0, cus, num_splits))
+
+
+def _ranges(plan, n_kv):
+    """First and last key of every range of a launch."""
+    per = plan["split_tiles"] * plan["keys"] or n_kv
+    return [(x, min(x + per, n_kv)) for x in range(0, n_kv, per)]
+
+
+def _calls(n, seed):
+    rnd = random.Random(seed)
+    for _ in range(n):
+        h_kv, group = rnd.choice([1, 2, 4, 8, 16]), rnd.choice([1, 1, 2, 4, 5, 7, 8, 16, 56])
+        yield (rnd.choice([1, 1, 2, 3, 8, 20]), h_kv * group, h_kv, rnd.choice([1, 1, 2, 7, 16, 40, 150, 700]),
+               rnd.choice([1, 100, 129, 513, 1000, 1088, 1536, 2112, 3000, 4097, 8192, 16483, 32000, 40001]),
+               rnd.choice([16, 32, 64, 128]))
+
+
+@needs_ablate
+@pytest.mark.parametrize("cus,xcds", [(256, 8), (304, 8), (96, 4)])
+def test_launch_splits_is_the_count_that_runs(cus, xcds):
+    """Over key counts that are no multiple of a tile and every num_splits: the count told is the
+    count of the plan, passing it back makes the same ranges with its own workspace, and every range
+    holds keys. A workspace of the requested count, and of the least count accepted."""
+    lib = _lib.lib()
+    seen = set()
+    for sizes in _calls(500, cus):
+        B, h_q, h_kv, n_q, n_kv, D = sizes
+        for n in (2, 3, 5, 7, 8, 12, 16):
+            told = _launch_splits(*sizes, n, cus)
+            ws = lib.fa2_workspace_bytes(B, h_q, n_q, D, n)
+            plan = _plan(*sizes, 0, False, num_splits=n, workspace_bytes=ws, cus=cus, xcds=xcds)
+            assert told == plan["splits"], (sizes, n, told, plan)
+            again = _plan(*sizes, 0, False, num_splits=told, cus=cus, xcds=xcds,
+                          workspace_bytes=lib.fa2_workspace_bytes(B, h_q, n_q, D, told))
+            assert again == plan and _launch_splits(*sizes, told, cus) == told, (sizes, n, plan, again)
+            assert len(_ranges(plan, n_kv)) == told <= n
+            seen.add((plan["kernel"], told))
+            # the least workspace accepted holds the general kernel's ranges: no kernel runs more
+            tiles = -(-n_kv // (128 if D == 16 else 64))
+            least = -(-tiles // -(-tiles // n))
+            if least > 1:
+                tight = _plan(*sizes, 0, False, num_splits=n, cus=cus, xcds=xcds,
+                              workspace_bytes=lib.fa2_workspace_bytes(B, h_q, n_q, D, least))
+                assert tight == plan and plan["splits"] <= least
+                with pytest.raises(RuntimeError, match="workspace"):
+                    _plan(*sizes, 0, False, num_splits=n, cus=cus, xcds=xcds,
+                          workspace_bytes=lib.fa2_workspace_bytes(B, h_q, n_q, D, least) - 256)
+    assert len({k for k, _ in seen}) == 2 and {k for k, s in seen if s > 8} >= {WAVE_SPLIT}
+
+
+@needs_ablate
+@pytest.mark.parametrize("n_kv,n,want", [(1088, 16, 6), (1088, 8, 6), (1088, 6, 6), (2112, 16, 11),
+                                         (2112, 12, 11), (4096, 16, 16), (4096, 3, 3)])
+def test_wave_split_ranges(n_kv, n, want):
+    """B1 H32/8 head_dim 128, one query, 32-key tiles: ranges of whole pairs of them (1088 keys are 17
+    pairs; eight ranges of three are six), whatever larger count was asked for."""
+    plan = _plan(1, 32, 8, 1, n_kv, 128, 1, False, num_splits=n,
+                 workspace_bytes=_lib.lib().fa2_workspace_bytes(1, 32, 1, 128, n))
+    assert plan["kernel"] == WAVE_SPLIT and plan["keys"] == 32 and plan["splits"] == want
+    assert plan["split_tiles"] % 2 == 0
+    assert _launch_splits(1, 32, 8, 1, n_kv, 128, n) == want
+
+
+@needs_ablate
+def test_default_count_covers_what_the_launch_runs():
+    """fa2_num_splits: the workspace of its count is accepted, and a larger one changes nothing."""
+    lib = _lib.lib()
+    for sizes in _calls(600, 5):
+        B, h_q, h_kv, n_q, n_kv, D = sizes
+        n = _lib.num_splits(*sizes, False, 128, 0, 256)
+        ws = lib.fa2_workspace_bytes(B, h_q, n_q, D, n)
+        plan = _plan(*sizes, 0, False, num_splits=n, workspace_bytes=ws)
+        assert plan["splits"] <= n
+        if plan["kernel"] == WAVE_SPLIT:
+            more = _plan(*sizes, 0, False, num_splits=16,
+                         workspace_bytes=lib.fa2_workspace_bytes(B, h_q, n_q, D, 16))
+            assert more == plan, (sizes, plan, more)

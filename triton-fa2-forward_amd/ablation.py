@@ -102,10 +102,30 @@ def ablate_lib():
         lib.fa2_ablate_attn_fwd.restype = ctypes.c_int
         lib.fa2_ablate_attn_fwd.argtypes = [vp, vp, vp, vp, i64p, i64p, i64p, i64p] + [i32] * 9 + \
             [ctypes.c_float, i32, vp]
+        lib.fa2_ablate_plan.restype = ctypes.c_int
+        lib.fa2_ablate_plan.argtypes = [i32] * 12 + [ctypes.c_size_t, i32, i32, ctypes.POINTER(i32), i32]
         lib.fa2_ablate_last_error.restype = ctypes.c_char_p
         lib.fa2_ablate_last_error.argtypes = []
         _LIB = lib
     return _LIB
+
+
+KERNELS = ("fa2::attn_fwd_kernel", "fa2::attn_wave_split_kernel", "fa2::attn_wide_kernel")
+
+
+def launch_plan(B, H_q, H_kv, N_q, N_kv, D, dtype_code, causal, *, pack=1, block_m=128, block_n=0,
+                num_splits=1, workspace_bytes=0, cus=256, xcds=8):
+    """What fa2_attn_fwd_ex launches for a call of these sizes (fa2_ablate_plan; no GPU call): its
+    kernel, rows per workgroup, keys per tile, splits, tiles per split, workgroups, key-norm table."""
+    info = (ctypes.c_int32 * 7)()
+    lib = ablate_lib()
+    rc = lib.fa2_ablate_plan(B, H_q, H_kv, N_q, N_kv, D, dtype_code, int(bool(causal)), pack, block_m,
+                             block_n, num_splits, workspace_bytes, cus, xcds, info, len(info))
+    if rc != 0:
+        raise RuntimeError(f"fa2_ablate_plan failed ({rc}): "
+                           f"{lib.fa2_ablate_last_error().decode(errors='replace')}")
+    return {"kernel": KERNELS[info[0]], "rows": info[1], "keys": info[2], "splits": info[3],
+            "split_tiles": info[4], "grid": info[5], "key_table": bool(info[6])}
 
 
 def variant_bits(switches):

@@ -108,7 +108,7 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
 
 // The kernel choice of a call at the default tiles: the wave-split kernel (attn_fwd_wavesplit.hpp)
 // with 32 * row_waves rows a workgroup and `splits` key ranges, or the general kernel
-// (row_waves 0). Independent of pack, as packed and unpacked calls must agree bit for bit.
+// (row_waves 0; its split count is its caller's). Independent of pack, as packed and unpacked calls must agree bit for bit.
 //
 // The wave-split kernel walks a row's keys with 4 / row_waves waves at once, which shortens a
 // launch that its longest key range bounds, but it stages K/V into LDS two or four times as often
@@ -159,10 +159,8 @@ struct KernelChoice {
   int row_waves = 0, splits = 1;
 };
 KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64_t n_kv,
-                           int32_t head_dim, bool causal, int32_t block_m, int32_t bn, int cus,
-                           int max_splits) {
+                           int32_t head_dim, bool causal, int32_t block_m, int32_t bn, int cus) {
   KernelChoice kc;
-  kc.splits = max_splits;  // the general kernel takes the count it is given
   if (block_m != 128 || bn != default_block_n(head_dim)) return kc;
   const int64_t rows = n_q * (h_q / h_kv), units = batch * h_kv;
   if (n_kv <= (head_dim == 128 && (causal || rows > 32) ? 192 : 128)) return kc;
@@ -179,12 +177,11 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
   // 128-key tiles of D16 and D32 take about twice as long each: D16 MQA B4 2000 keys (3.9 tiles) 8.1
   // 8.1 7.3 7.7 8.3.
   auto take_splits = [&]() {
-    kc.splits = 1;
     const int step = 4 * fa2::wave_split_block_n(head_dim, 1, false);
     const int64_t tiles = n_kv / step;  // ... a wave walks without splits
     const int64_t least = (4 * w1 <= cus ? 7 : 14) * (int64_t)step / (small ? 2 : 1);
     if (n_kv >= least)
-      while (kc.splits * 2 <= max_splits && w1 * kc.splits * 2 <= cus && tiles / kc.splits >= 2)
+      while (kc.splits * 2 <= kMaxSplits && w1 * kc.splits * 2 <= cus && tiles / kc.splits >= 2)
         kc.splits *= 2;
   };
   if (causal) {  // (num_splits is 1)
@@ -201,7 +198,6 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
       return kc;
     }
     // more 32-row workgroups than CUs (the first list above)
-    kc.splits = 1;
     if (rows > 32) {
       bool general;  // where it packs: its one 128-row program is as good or better
       if (head_dim == 128)
@@ -219,7 +215,6 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
     } else if (n_kv < 320 || (n_kv < 768 && w1 > 2 * cus)) {
       kc.row_waves = 2;
     }
-    if (!kc.row_waves) kc.splits = max_splits;
   } else if (n_kv <= (head_dim == 128 ? 2048 : 4096)) {
     if (w1 <= cus) {
       kc.row_waves = 1;
@@ -227,16 +222,11 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
     } else if (w1 <= 2 * cus && n_kv >= (small ? 512 : 0)) {
       // two workgroups on some CUs: 64 rows a workgroup where that still reaches every CU
       kc.row_waves = 10 * w2 >= 9 * cus ? 2 : 1;
-      kc.splits = 1;
     } else if (head_dim == 32 && w2 <= 2 * cus && n_kv >= 512) {
       kc.row_waves = 2;
-      kc.splits = 1;
     }
   }
-  if (!causal && small && n_kv >= 512 && w2 > 2 * cus && w2 <= 3 * cus) {
-    kc.row_waves = 2;
-    kc.splits = 1;
-  }
+  if (!causal && small && n_kv >= 512 && w2 > 2 * cus && w2 <= 3 * cus) kc.row_waves = 2;
   if (!causal && !kc.row_waves && !packs && rows > 64) {
     // 64-row slots the general kernel fills, of one query head each, against the rows' own
     const int64_t slots = (n_q + 127) / 128 * 2 * (h_q / h_kv) * units;
@@ -244,9 +234,8 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
       if (2 * slots >= 3 * w2) {
         if (!small && n_kv >= 6144 && 2 * w1 > cus) {
           kc.row_waves = 2;
-          kc.splits = 1;
           const int64_t tiles = n_kv / (2 * fa2::wave_split_block_n(head_dim, 2, false));
-          while (kc.splits * 2 <= max_splits && w2 * kc.splits <= cus && tiles / kc.splits >= 8)
+          while (kc.splits * 2 <= kMaxSplits && w2 * kc.splits <= cus && tiles / kc.splits >= 8)
             kc.splits *= 2;
         } else {
           kc.row_waves = 1;
@@ -255,10 +244,52 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
       }
     } else if (2 * slots >= (n_kv >= 512 ? 3 : 5) * w2) {
       kc.row_waves = 2;
-      kc.splits = 1;
     }
   }
   return kc;
+}
+
+// Key ranges of whole tiles that `tiles` are cut into when n are asked for: none is empty.
+int clamp_splits(int64_t tiles, int n) {
+  const int64_t per = (tiles + n - 1) / n;
+  return (int)((tiles + per - 1) / per);
+}
+
+// The kernel of a launch given num_splits and the key ranges it runs: plan_launch's choice, and what
+// fa2_launch_splits tells. The wave-split kernel takes its own count, at most num_splits, the general
+// kernel the count it is given. Ranges are whole tiles of the wider of the two kernels' tiles: at
+// head_dim 128 an even number of 32-key tiles, as an odd one leaves a wave of the last round alone
+// (B2 H32/8, one query of 2112 keys: 11 ranges of 6 tiles 9.8 us, 14 of 5 10.5 us), and never more
+// ranges than the general kernel's, whose partials the workspace must hold. A launch given the count
+// that runs makes the same ranges: clamp_splits(t, clamp_splits(t, n)) == clamp_splits(t, n).
+struct SplitChoice {
+  int row_waves = 0;    // > 0: the wave-split kernel
+  int splits = 1;
+  int split_tiles = 0;  // tiles, of the kernel that runs, per range; 0 for one range
+  int need = 1;         // the workspace must hold the partials of this many ranges
+};
+SplitChoice split_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64_t n_kv,
+                         int32_t head_dim, bool causal, int32_t block_m, int32_t bn, int cus,
+                         int num_splits, bool general_only) {
+  SplitChoice sc;
+  int own = bn, n = num_splits;  // keys per tile of the kernel that runs; ranges it asks for
+  if (n > 1 && n_kv > 0) sc.need = clamp_splits((n_kv + bn - 1) / bn, n);
+  if (!general_only) {
+    const KernelChoice kc =
+        kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, causal, block_m, bn, cus);
+    if (kc.row_waves) {
+      sc.row_waves = kc.row_waves;
+      own = fa2::wave_split_block_n(head_dim, kc.row_waves, causal);
+      n = std::min(n, kc.splits);
+    }
+  }
+  if (n > 1 && n_kv > 0) {
+    const int unit = std::max(own, bn);
+    const int64_t units = (n_kv + unit - 1) / unit;
+    sc.splits = clamp_splits(units, n);
+    if (sc.splits > 1) sc.split_tiles = (int)((units + sc.splits - 1) / sc.splits) * (unit / own);
+  }
+  return sc;
 }
 
 // Whether a full (not causal) call at the default tiles runs the wide kernel (attn_fwd_wide.hpp),
@@ -749,21 +780,16 @@ int plan_launch(const LaunchArgs& a, const Topology& topo, LaunchPlan* out,
 
   // The kernel: the general one, or the wave-split one, whose rows are a KV head's whole group
   // whatever pack. A caller that brings the table's room asks for the instance that uses it.
-  int kv_bn = bn;
-  int splits = a.num_splits;
-  if (!table_room && !a.general_only &&
-      (a.variant == 0 || a.variant == fa2::kVariantMaskEveryTile)) {
-    const KernelChoice kc =
-        kernel_choice(a.batch, a.h_q, a.h_kv, a.n_q, a.n_kv, a.head_dim, a.causal != 0, a.block_m,
-                      bn, topo.cus, a.num_splits);
-    if (kc.row_waves) {
-      pl.row_waves = kc.row_waves;
-      splits = kc.splits;
-      kv_bn = fa2::wave_split_block_n(a.head_dim, kc.row_waves, a.causal != 0);
-      const int64_t tile_rows = 32 * kc.row_waves;
-      p.n_tiles = (int32_t)(((int64_t)a.n_q * group + tile_rows - 1) / tile_rows);
-      p.n_bh = (int32_t)((int64_t)a.batch * a.h_kv);
-    }
+  const bool general_only = table_room || a.general_only ||
+                            (a.variant != 0 && a.variant != fa2::kVariantMaskEveryTile);
+  const SplitChoice sc = split_choice(a.batch, a.h_q, a.h_kv, a.n_q, a.n_kv, a.head_dim,
+                                      a.causal != 0, a.block_m, bn, topo.cus, a.num_splits,
+                                      general_only);
+  if (sc.row_waves) {
+    pl.row_waves = sc.row_waves;
+    const int64_t tile_rows = 32 * sc.row_waves;
+    p.n_tiles = (int32_t)(((int64_t)a.n_q * group + tile_rows - 1) / tile_rows);
+    p.n_bh = (int32_t)((int64_t)a.batch * a.h_kv);
   }
 
   if (a.wide_ok && !pl.row_waves && a.num_splits == 1 && a.block_m == 128 && bn == 64 && !a.causal &&
@@ -772,21 +798,9 @@ int plan_launch(const LaunchArgs& a, const Topology& topo, LaunchPlan* out,
     p.n_tiles = (int32_t)((rows + fa2::kWideRows - 1) / fa2::kWideRows);
   }
 
-  // Split-KV: cut the key range into whole tiles; drop splits that would be empty. The workspace
-  // must hold the partials of the requested count at the general kernel's tiles, whichever kernel
-  // runs and however few splits it takes.
-  auto clamp_splits = [](int64_t tiles, int n) {
-    const int64_t per = (tiles + n - 1) / n;
-    return (int)((tiles + per - 1) / per);
-  };
-  const int need =
-      a.num_splits > 1 && a.n_kv > 0 ? clamp_splits(((int64_t)a.n_kv + bn - 1) / bn, a.num_splits) : 1;
-  splits = std::min(splits, need);
-  if (splits > 1) {
-    const int64_t kv_tiles = ((int64_t)a.n_kv + kv_bn - 1) / kv_bn;
-    p.split_tiles = (int32_t)((kv_tiles + splits - 1) / splits);
-    splits = clamp_splits(kv_tiles, splits);
-  }
+  // Split-KV: the key range in whole tiles, without empty splits. The workspace must hold the
+  // partials of the requested count at the general kernel's tiles, whichever kernel runs.
+  const int splits = sc.splits, need = sc.need;
   if (need > 1) {
     const WorkspaceLayout w = workspace_layout((size_t)p.part_rows, a.head_dim, need);
     if (!a.workspace || a.workspace_bytes < w.total)
@@ -804,8 +818,7 @@ int plan_launch(const LaunchArgs& a, const Topology& topo, LaunchPlan* out,
     p.part_lse = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + w.part_lse);
     p.part_lse_exact = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + w.part_lse_exact);
     p.splits = splits;
-  } else {
-    p.split_tiles = 0;
+    p.split_tiles = sc.split_tiles;
   }
   int64_t grid = (int64_t)p.n_tiles * p.n_bh * splits;
   if (grid > 0x7fffffffLL)

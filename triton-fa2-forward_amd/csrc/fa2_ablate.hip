@@ -196,6 +196,40 @@ int fa2_ablate_program_map(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q
   return 0;
 }
 
+int fa2_ablate_plan(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, int32_t n_kv,
+                    int32_t head_dim, int32_t dtype, int32_t causal, int32_t pack, int32_t block_m,
+                    int32_t block_n, int32_t num_splits, size_t workspace_bytes, int32_t cus,
+                    int32_t xcds, int32_t* info, int32_t info_words) {
+  g_err[0] = '\0';
+  if (!info || info_words < FA2_ABLATE_PLAN_INFO_WORDS)
+    return fail(FA2_EINVAL, "info needs %d words", FA2_ABLATE_PLAN_INFO_WORDS);
+  const int64_t d = head_dim, q = n_q, k = n_kv;
+  const int64_t sq[4] = {h_q * q * d, q * d, d, 1};
+  const int64_t sk[4] = {h_kv * k * d, k * d, d, 1};
+  // stand-in device addresses: the plan checks their alignment and never dereferences them
+  void* const fake = reinterpret_cast<void*>(uintptr_t(1) << 20);
+  LaunchArgs a{fake, fake, fake, fake, sq, sk, sk, sq, batch, h_q, h_kv, n_q, n_kv,
+               head_dim, dtype, causal, pack, block_m, block_n, 1.0f, nullptr, num_splits,
+               workspace_bytes ? fake : nullptr, workspace_bytes, 0, nullptr, 0, false};
+  a.wide_ok = true;
+  LaunchPlan pl;
+  const int rc = plan_launch(a, make_topology(cus, xcds), &pl);
+  if (rc != FA2_OK) return rc;
+  if (pl.empty) {
+    for (int i = 0; i < FA2_ABLATE_PLAN_INFO_WORDS; ++i) info[i] = 0;
+    return FA2_OK;
+  }
+  const bool wide = pl.p.block_m != block_m;  // the wide kernel's programs have their own rows
+  const int32_t vals[FA2_ABLATE_PLAN_INFO_WORDS] = {
+      pl.row_waves ? 1 : wide ? 2 : 0,
+      pl.row_waves ? 32 * pl.row_waves : pl.p.block_m,
+      pl.row_waves ? fa2::wave_split_block_n(head_dim, pl.row_waves, causal != 0) : pl.bn,
+      pl.splits, pl.splits > 1 ? pl.p.split_tiles : 0, (int32_t)pl.grid,
+      pl.key_table ? 1 : 0};
+  for (int i = 0; i < FA2_ABLATE_PLAN_INFO_WORDS; ++i) info[i] = vals[i];
+  return FA2_OK;
+}
+
 long long fa2_ablate_tail_launches(void) { return g_tail_launches.load(); }
 
 int fa2_ablate_mfma_ceiling(int32_t mode, int32_t workgroups, int32_t iters, float* out,

@@ -115,8 +115,8 @@ int32_t fa2_num_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, in
   // it is smaller the launch itself takes fewer than it is given.)
   int s = 1;
   while (programs * s < num_cus && s * 2 <= kMaxSplits && tiles / (s * 2) >= kMinSplitTiles) s *= 2;
-  const KernelChoice kc = kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, false, block_m, bn,
-                                        num_cus, kMaxSplits);
+  const KernelChoice kc =
+      kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, false, block_m, bn, num_cus);
   return kc.row_waves ? std::max(s, kc.splits) : s;
 }
 
@@ -126,8 +126,8 @@ int32_t fa2_launch_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q,
   if (num_splits <= 1 || causal || batch <= 0 || h_q <= 0 || h_kv <= 0 || h_q % h_kv || n_q <= 0 ||
       n_kv <= 0 || block_m <= 0 || num_cus <= 0 || dim_index(head_dim) < 0)
     return num_splits;
-  return kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, false, block_m,
-                       tile_n(block_n, head_dim), num_cus, num_splits).splits;
+  return split_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, false, block_m,
+                      tile_n(block_n, head_dim), num_cus, num_splits, false).splits;
 }
 
 int fa2_attn_fwd_ex(const void* q, const void* k, const void* v, void* out,
