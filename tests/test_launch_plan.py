@@ -1,5 +1,5 @@
 """The split counts the library tells against the ones it runs, on the CPU: fa2_launch_splits and
-fa2_num_splits (include/fa2_fwd.h) against the plan of the launch itself (fa2_ablate_plan: the
+fa2_num_splits (include/fa2_fwd.h) and the native call's policy against the plan of the launch itself (fa2_ablate_plan: the
 library's planning code, without a GPU call).
 """
 
@@ -72,14 +72,13 @@ def test_launch_splits_is_the_count_that_runs(cus, xcds):
 
 @needs_ablate
 @pytest.mark.parametrize("n_kv,n,want", [(1088, 16, 6), (1088, 8, 6), (1088, 6, 6), (2112, 16, 11),
-                                         (2112, 12, 11), (4096, 16, 16), (4096, 3, 3)])
+                                         (2112, 12, 11), (4096, 16, 16), (4096, 3, 3), (31987, 16, 16)])
 def test_wave_split_ranges(n_kv, n, want):
-    """B1 H32/8 head_dim 128, one query, 32-key tiles: ranges of whole pairs of them (1088 keys are 17
-    pairs; eight ranges of three are six), whatever larger count was asked for."""
+    """B1 H32/8 head_dim 128, one query, 32-key tiles: the count that leaves no range empty in them and
+    in 64-key tiles (1088 keys are 34 or 17 of them), whatever larger count was asked for."""
     plan = _plan(1, 32, 8, 1, n_kv, 128, 1, False, num_splits=n,
                  workspace_bytes=_lib.lib().fa2_workspace_bytes(1, 32, 1, 128, n))
     assert plan["kernel"] == WAVE_SPLIT and plan["keys"] == 32 and plan["splits"] == want
-    assert plan["split_tiles"] % 2 == 0
     assert _launch_splits(1, 32, 8, 1, n_kv, 128, n) == want
 
 

@@ -257,11 +257,13 @@ int clamp_splits(int64_t tiles, int n) {
 
 // The kernel of a launch given num_splits and the key ranges it runs: plan_launch's choice, and what
 // fa2_launch_splits tells. The wave-split kernel takes its own count, at most num_splits, the general
-// kernel the count it is given. Ranges are whole tiles of the wider of the two kernels' tiles: at
-// head_dim 128 an even number of 32-key tiles, as an odd one leaves a wave of the last round alone
-// (B2 H32/8, one query of 2112 keys: 11 ranges of 6 tiles 9.8 us, 14 of 5 10.5 us), and never more
-// ranges than the general kernel's, whose partials the workspace must hold. A launch given the count
-// that runs makes the same ranges: clamp_splits(t, clamp_splits(t, n)) == clamp_splits(t, n).
+// kernel the count it is given; either way the largest count, from there down, that leaves no range
+// empty in the tiles of both kernels. So a launch given the count that runs makes the same ranges,
+// there are never more of them than the general kernel's, whose partials the workspace must hold.
+// Counting in the general kernel's 64-key tiles as well is faster where ranges are short (head_dim 128,
+// 32-key tiles, B2 H32/8, one query of 2112 keys: 11 ranges of 6 tiles 9.8 us, 14 of 5 10.5 us); the
+// ranges are then cut in the kernel's own tiles (B1 H32/8, one query of 31987 keys: 16 of 63 31.1 us,
+// 16 of 64, all 512 KiB apart, 32.8 us).
 struct SplitChoice {
   int row_waves = 0;    // > 0: the wave-split kernel
   int splits = 1;
@@ -284,10 +286,12 @@ SplitChoice split_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, 
     }
   }
   if (n > 1 && n_kv > 0) {
-    const int unit = std::max(own, bn);
-    const int64_t units = (n_kv + unit - 1) / unit;
-    sc.splits = clamp_splits(units, n);
-    if (sc.splits > 1) sc.split_tiles = (int)((units + sc.splits - 1) / sc.splits) * (unit / own);
+    const int64_t tiles = (n_kv + own - 1) / own, general_tiles = (n_kv + bn - 1) / bn;
+    do {
+      sc.splits = n;
+      n = clamp_splits(tiles, clamp_splits(general_tiles, n));
+    } while (n < sc.splits);
+    if (n > 1) sc.split_tiles = (int)((tiles + n - 1) / n);
   }
   return sc;
 }
