@@ -52,6 +52,14 @@ def test_same_bits_as_python(both, dtype, lse, shape, causal):
                 assert torch.equal(a, b) and a.dtype == b.dtype and a.stride() == b.stride()
 
 
+def test_same_bits_where_the_key_norm_table_keeps_the_split_count(both):
+    """A group of 56 does not pack into 128 rows: without the table the wave-split kernel would take
+    two splits; with it (bf16, long keys) the general kernel takes all four asked for."""
+    native, python = both
+    q, k, v = make_qkv(1, 56, 1, 150, 32768, 128, torch.bfloat16)
+    assert torch.equal(native(q, k, v, False, None, False), python(q, k, v, causal=False))
+
+
 def test_side_stream_and_grad(both):
     native, python = both
     q, k, v = make_qkv(1, 8, 2, 500, 500, 64, torch.bfloat16)

@@ -96,3 +96,31 @@ def test_default_count_covers_what_the_launch_runs():
             more = _plan(*sizes, 0, False, num_splits=16,
                          workspace_bytes=lib.fa2_workspace_bytes(B, h_q, n_q, D, 16))
             assert more == plan, (sizes, plan, more)
+
+
+@needs_ablate
+def test_native_call_plans_attentions_launch():
+    """The native call's packing, splits and workspace (fa2/_torch_call.so) give the launch that
+    attention()'s Python gives with fa2_num_splits's count, also where the key-norm table pays and the
+    wave-split kernel would take fewer splits (B1 H56/1, 150 queries of 32768 keys in bf16)."""
+    from fa2._torch_call import policy
+    from fa2.kernel import should_pack_gqa
+
+    lib = _lib.lib()
+    calls = list(_calls(1500, 7)) + [(1, g, 1, n_q, n_kv, D) for g in (48, 56, 60) for D in (64, 128)
+                                     for n_q in (130, 150, 170) for n_kv in (8192, 32768, 65536)]
+    tables = 0
+    for sizes in calls:
+        B, h_q, h_kv, n_q, n_kv, D = sizes
+        for dtype in (0, 1):
+            for causal in (False, True) if n_q == n_kv else (False,):
+                n = 1 if causal else _lib.num_splits(*sizes, causal, 128, 0, 256)
+                ws = lib.fa2_workspace_bytes_for(*sizes, dtype, int(causal), n)
+                pack = h_q // h_kv if should_pack_gqa(n_q, h_q // h_kv, 128) else 1
+                want = _plan(*sizes, dtype, causal, pack=pack, num_splits=n, workspace_bytes=ws)
+                got_pack, got_n, got_ws = policy(*sizes, dtype, int(causal), 256)
+                got = _plan(*sizes, dtype, causal, pack=got_pack, num_splits=got_n, workspace_bytes=got_ws)
+                assert got == want and got_pack == pack and got_ws <= ws, (sizes, dtype, want, got)
+                tables += want["key_table"] and n > _launch_splits(*sizes, n)
+    assert tables >= 3
+    assert policy(1, 56, 1, 150, 32768, 128, 1, 0, 256)[1] == 4

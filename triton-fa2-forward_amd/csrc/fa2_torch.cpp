@@ -71,6 +71,43 @@ bool strides_of(const at::Tensor& t, int64_t max_row, int64_t (&s)[4]) {
   return s[2] <= max_row;
 }
 
+// attention()'s policy at the default tiles: packing, split count and workspace. The count is the one
+// that runs, which needs the smaller workspace, unless the workspace has room for the key-norm table:
+// the kernel that uses the table takes fa2_num_splits's count, as fa2_launch_splits's contract says.
+struct Policy {
+  int32_t bm = 0, bn = 0, pack = 1, splits = 1;
+  size_t ws_bytes = 0;
+};
+bool policy_of(int32_t B, int32_t hq, int32_t hkv, int32_t nq, int32_t nkv, int32_t D, int32_t dtype,
+               int32_t causal, int32_t cus, Policy* out) {
+  Policy p;
+  if (fa2_default_config(D, &p.bm, &p.bn, nullptr, nullptr) != FA2_OK) return false;
+  if (fa2_should_pack_gqa(nq, hq / hkv, p.bm)) p.pack = hq / hkv;
+  if (!causal) p.splits = fa2_num_splits(B, hq, hkv, nq, nkv, D, 0, p.bm, p.bn, cus);
+  p.ws_bytes = fa2_workspace_bytes_for(B, hq, hkv, nq, nkv, D, dtype, causal, p.splits);
+  if (p.splits > 1 && p.ws_bytes == fa2_workspace_bytes(B, hq, nq, D, p.splits)) {
+    p.splits = fa2_launch_splits(B, hq, hkv, nq, nkv, D, 0, p.bm, p.bn, cus, p.splits);
+    p.ws_bytes = fa2_workspace_bytes(B, hq, nq, D, p.splits);
+  }
+  *out = p;
+  return true;
+}
+
+// policy(batch, h_q, h_kv, n_q, n_kv, head_dim, dtype, causal, cus) -> (pack, splits, workspace bytes)
+// of a call of these sizes on a GPU of `cus` CUs (dtype: the C ABI's code). No GPU call.
+PyObject* policy(PyObject*, PyObject* args) {
+  int B, hq, hkv, nq, nkv, D, dtype, causal, cus;
+  if (!PyArg_ParseTuple(args, "iiiiiiiii", &B, &hq, &hkv, &nq, &nkv, &D, &dtype, &causal, &cus))
+    return nullptr;
+  Policy p;
+  if (B < 1 || hkv < 1 || hq < 1 || hq % hkv || nq < 1 || nkv < 1 || cus < 1 ||
+      !policy_of(B, hq, hkv, nq, nkv, D, dtype, causal, cus, &p)) {
+    PyErr_SetString(PyExc_ValueError, "sizes that attention() rejects");
+    return nullptr;
+  }
+  return Py_BuildValue("iin", p.pack, p.splits, (Py_ssize_t)p.ws_bytes);
+}
+
 // call(q, k, v, causal, sm_scale, return_lse) -> attention()'s result, or None (see above)
 PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
@@ -113,42 +150,30 @@ PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
       !strides_of(v, kMaxKvRowStride, sv))
     Py_RETURN_NONE;
 
-  // ---- its policy: default tiles, packing and split count
-  int32_t bm = 0, bn = 0;
-  if (fa2_default_config((int32_t)D, &bm, &bn, nullptr, nullptr) != FA2_OK) Py_RETURN_NONE;
-  const int32_t group = (int32_t)(hq / hkv);
-  if (nq > INT32_MAX / group) Py_RETURN_NONE;
-  const int32_t pack = fa2_should_pack_gqa((int32_t)nq, group, bm) ? group : 1;
+  const int cus = causal ? 1 : cu_count(device.index());
   const int32_t code = dtype == at::kBFloat16 ? FA2_DTYPE_BF16 : FA2_DTYPE_F16;
-  int32_t splits = 1;
-  if (!causal) {
-    const int cus = cu_count(device.index());
-    if (cus < 1) Py_RETURN_NONE;
-    splits = fa2_num_splits((int32_t)B, (int32_t)hq, (int32_t)hkv, (int32_t)nq, (int32_t)nkv,
-                            (int32_t)D, 0, bm, bn, cus);
-    splits = fa2_launch_splits((int32_t)B, (int32_t)hq, (int32_t)hkv, (int32_t)nq, (int32_t)nkv,
-                               (int32_t)D, 0, bm, bn, cus, splits);
-  }
+  Policy p;
+  if (cus < 1 || nq > INT32_MAX / (hq / hkv) ||
+      !policy_of((int32_t)B, (int32_t)hq, (int32_t)hkv, (int32_t)nq, (int32_t)nkv, (int32_t)D, code,
+                 causal, cus, &p))
+    Py_RETURN_NONE;
 
   // ---- outputs, workspace, launch
   at::Tensor out = at::empty_like(q);
   if (!strides_of(out, INT64_MAX, so)) Py_RETURN_NONE;
   at::Tensor lse, ws;
   if (want_lse) lse = at::empty({B, hq, nq}, q.options().dtype(at::kFloat));
-  const size_t ws_bytes =
-      fa2_workspace_bytes_for((int32_t)B, (int32_t)hq, (int32_t)hkv, (int32_t)nq, (int32_t)nkv,
-                              (int32_t)D, code, causal, splits);
-  if (ws_bytes) ws = at::empty({(int64_t)ws_bytes}, q.options().dtype(at::kByte));
+  if (p.ws_bytes) ws = at::empty({(int64_t)p.ws_bytes}, q.options().dtype(at::kByte));
   void* stream = c10::hip::getCurrentHIPStream(device.index()).stream();
   const void *qp = q.data_ptr(), *kp = k.data_ptr(), *vp = v.data_ptr();
   void* op = out.data_ptr();
   float* lp = want_lse ? static_cast<float*>(lse.data_ptr()) : nullptr;
-  void* wp = ws_bytes ? ws.data_ptr() : nullptr;
+  void* wp = p.ws_bytes ? ws.data_ptr() : nullptr;
   int rc;
   Py_BEGIN_ALLOW_THREADS  // as ctypes does around a foreign call
   rc = fa2_attn_fwd_ex(qp, kp, vp, op, sq, sk, sv, so, (int32_t)B, (int32_t)hq, (int32_t)hkv,
-                       (int32_t)nq, (int32_t)nkv, (int32_t)D, code, causal, pack, bm, bn,
-                       (float)(sm_scale * kLog2e), lp, splits, wp, ws_bytes, stream);
+                       (int32_t)nq, (int32_t)nkv, (int32_t)D, code, causal, p.pack, p.bm, p.bn,
+                       (float)(sm_scale * kLog2e), lp, p.splits, wp, p.ws_bytes, stream);
   Py_END_ALLOW_THREADS
   if (rc != FA2_OK) Py_RETURN_NONE;  // nothing ran: attention() repeats the call and raises
   PyObject* o = THPVariable_Wrap(std::move(out));
@@ -168,6 +193,8 @@ PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
 PyMethodDef methods[] = {
     {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(call)), METH_FASTCALL,
      "call(q, k, v, causal, sm_scale, return_lse) -> attention()'s result, or None"},
+    {"policy", policy, METH_VARARGS,
+     "policy(batch, h_q, h_kv, n_q, n_kv, head_dim, dtype, causal, cus) -> (pack, splits, workspace bytes)"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_call", nullptr, -1, methods,
                       nullptr, nullptr, nullptr, nullptr};
