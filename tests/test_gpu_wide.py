@@ -50,6 +50,24 @@ def test_same_bits_as_the_general_kernel(dtype, D, table, B, h_q, h_kv, n, n_kv)
         check_against_oracle(q, k, v, False, precision=torch.float32, ours=out)
 
 
+# shapes that run the wide kernel at both head dims: one round of programs per CU place at 32, ragged
+# last programs and key tiles, a grouped and an unpackable head count
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("table", [False, True])
+@pytest.mark.parametrize("B,h_q,h_kv,n,n_kv", [(12, 16, 16, 1024, 1024), (3, 32, 8, 2047, 1025),
+                                               (15, 16, 4, 1000, 1500), (1, 16, 16, 15700, 1090)])
+def test_same_bits_where_the_wide_kernel_runs(dtype, D, table, B, h_q, h_kv, n, n_kv):
+    from ablation import launch_plan
+
+    plan = launch_plan(B, h_q, h_kv, n, n_kv, D, 0, False, workspace_bytes=1 << 30 if table else 0)
+    assert plan["kernel"] == "fa2::attn_wide_kernel" and plan["key_table"] == table
+    q, k, v = make_qkv(B, h_q, h_kv, n, n_kv, D, dtype)
+    k[:, 0] *= 3.0  # rows of this head fail the table's bound in fp16
+    k[:, -1] *= 0.3
+    _same_as_general(q, k, v, table)
+
+
 def test_reference_moves_on_every_tile_and_packed_rows():
     from fa2.kernel import attention
 

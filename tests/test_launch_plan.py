@@ -124,3 +124,22 @@ def test_native_call_plans_attentions_launch():
                 tables += want["key_table"] and n > _launch_splits(*sizes, n)
     assert tables >= 3
     assert policy(1, 56, 1, 150, 32768, 128, 1, 0, 256)[1] == 4
+
+
+# H16 on 256 CUs: batch and length, and whether 256-row programs pay. At head_dim 32 the launch lasts as
+# long as the CU with the most programs: 8 x 1024 is 2 per CU, 10 x 1024 2.5 (3 for 5 of 128 rows), 12 3,
+# 14 3.5 (4 for 7), 15 3.75, 18 4.5 (5 for 9), 28 7, 22 5.5 (6 for 11), 25 6.25 (7 for 13). At 64 it is
+# the last round of two per CU that matters. Rows past the last (3186) and short key ranges never pay.
+@needs_ablate
+@pytest.mark.parametrize("D,B,n,n_kv,wide", [
+    (32, 8, 1024, 1024, False), (32, 10, 1024, 1024, False), (32, 12, 1024, 1024, True),
+    (32, 14, 1024, 1024, False), (32, 15, 1024, 1024, True), (32, 18, 1024, 1024, False),
+    (32, 22, 1024, 1024, False), (32, 25, 1024, 1024, True), (32, 28, 1024, 1024, True),
+    (32, 12, 1024, 1000, False), (32, 12, 3186, 3186, False), (64, 8, 1024, 1024, True),
+    (64, 9, 1024, 1024, False), (64, 14, 1024, 1024, True), (64, 25, 1024, 1024, True),
+    (64, 12, 1024, 1000, False), (64, 12, 3186, 3186, False), (128, 12, 1024, 1024, False)])
+def test_wide_kernel_where_it_pays(D, B, n, n_kv, wide):
+    for dtype in (0, 1):
+        plan = _plan(B, 16, 16, n, n_kv, D, dtype, False)
+        assert (plan["kernel"] == "fa2::attn_wide_kernel") == wide, plan
+        assert not wide or plan["rows"] == 256

@@ -296,20 +296,31 @@ SplitChoice split_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, 
   return sc;
 }
 
-// Whether a full (not causal) call at the default tiles runs the wide kernel (attn_fwd_wide.hpp),
-// whose programs of 256 rows a CU holds two of: bit for bit the same output as the general kernel's
-// 128-row programs. Measured on MI355X (general -> wide, us; `rounds` of two programs per CU), H16 D64
-// unless stated: one round B8 N1024 45.3 -> 44.7, B4 N2048 82.9 -> 79.5, B2 N4096 156.0 -> 149.7; 1.5
-// B12 N1024 68.2 -> 66.6, 1.76 B5 H12 N3840 265.4 -> 253.0; 2 B4 N4096 305.6 -> 292.7; 3 B12 N2048
-// 237.7 -> 227.3, D32 160.6 -> 151.9. A last round that only a few programs reach costs more than that:
-// 1.12 rounds B3 H12 N4096 180.4 -> 199.8, 1.25 B5 N2048 101.4 -> 109.7; 0.75 B6 N1024 36.0 -> 40.4. So
-// do rows past the last (N3186: 13 programs of 256 rows for 24.9 of 128) 582.1 -> 590.2, and short key
-// ranges (B16 N512 27.6 -> 27.9).
+// Whether a full (not causal) call at the default tiles runs the wide kernel (attn_fwd_wide.hpp), whose
+// programs of 256 rows a CU holds two of at head_dim 64 and three of at 32 (tests/test_frontend.py holds
+// the compiler to it): bit for bit the same output as the general kernel's 128-row programs. Measured on
+// MI355X, general -> wide, us.
+//   * head_dim 64, in rounds of two programs per CU, H16 unless stated: one round B8 N1024 45.3 -> 44.7,
+//     B4 N2048 82.9 -> 79.5, B2 N4096 156.0 -> 149.7; 1.5 B12 N1024 68.2 -> 66.6, 1.76 B5 H12 N3840 265.4
+//     -> 253.0; 2 B4 N4096 305.6 -> 292.7; 3 B12 N2048 237.7 -> 227.3. A last round that only a few programs
+//     reach costs more than that: 1.12 rounds B3 H12 N4096 180.4 -> 199.8, 1.25 B5 N2048 101.4 -> 109.7;
+//     0.75 B6 N1024 36.0 -> 40.4. Rows past the last cost too (N3186: 13 programs of 256 rows for 24.9 of
+//     128) 582.1 -> 590.2, and so do short key ranges (B16 N512 27.6 -> 27.9).
+//   * head_dim 32 gains less, and a launch takes as long as the CUs with the most programs: two of the
+//     general kernel's there for each of these. Launches back to back, N1024 and N2048 H4 and H16, most
+//     programs per CU (twice the wide's / the general's): 6/5 +15-17% time, 6/6 -3..0%, 8/7 +7..11%, 8/8
+//     -4..+1%, 10/9 +5..8%, 10/10 -4..-1%, 12/11 0..+6%, 12/12 -6..-2%, 14/13 -3..+2%, 16/15 0..+1%, 16/16
+//     -2..-6%, 22/21 -1%. Two per CU leave one in three places of a CU empty: 4/4 +4..5% (N1024), 0..1%.
 bool wide_pays(int64_t rows, int64_t n_bh, int64_t n_kv, int32_t head_dim, int cus) {
   if ((head_dim != 32 && head_dim != 64) || n_kv < 1024) return false;
-  const int64_t tiles = (rows + fa2::kWideRows - 1) / fa2::kWideRows;
-  if (tiles * 2 * 100 > (rows + 127) / 128 * 102) return false;
-  const int64_t programs = tiles * n_bh, round = 2 * (int64_t)cus;
+  const int64_t tiles = (rows + fa2::kWideRows - 1) / fa2::kWideRows, general_tiles = (rows + 127) / 128;
+  if (tiles * 2 * 100 > general_tiles * 102) return false;
+  const int64_t programs = tiles * n_bh;
+  if (head_dim == 32) {
+    const int64_t most = (programs + cus - 1) / cus, general_most = (general_tiles * n_bh + cus - 1) / cus;
+    return most >= 3 && 13 * (2 * most) <= 14 * general_most;
+  }
+  const int64_t round = 2 * (int64_t)cus;
   const int64_t past = programs % round;  // programs of the last, partial round
   return programs >= round && (past == 0 || 10 * past >= 4 * round || programs >= 3 * round);
 }

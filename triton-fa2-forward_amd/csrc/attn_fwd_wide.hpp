@@ -10,11 +10,11 @@
 //     across a barrier, as the general kernel's pipelined loop needs);
 //   * every K and V operand read from LDS feeds two MFMAs instead of one, and a tile staged from L2
 //     serves 256 rows instead of 128.
-// Two waves per SIMD (214-220 VGPRs at head_dim 64), from two workgroups, so that their phases are
-// independent; the general kernel's 8-wave programs of 256 rows share a barrier instead, and lose.
+// Two waves per SIMD at head_dim 64 (214-220 VGPRs), three at 32 (155-161), each of another workgroup, so
+// that their phases are independent; the general kernel's 8-wave programs of 256 rows share a barrier instead, and lose.
 // Measured on MI355X against the general kernel (us, same box): fp16 full B2 H16 N16384 D64 at half
 // scale (key-norm table) 2198.5 -> 2078.3, bf16 2088.8 -> 1994.8; B8 H16 N2048 D64 162.5 -> 155.4;
-// D32 160.6 -> 151.9 (B12 N2048). Causal programs of 256 rows lose what this gains to their coarser
+// D32 164.3 -> 156.8 (fp16 B12 N2048). Causal programs of 256 rows lose what this gains to their coarser
 // tail (D64 B4 H16 N4096 162.6 -> 163.2, B2 86.4 -> 95.2), so there is no causal instance.
 #pragma once
 
