@@ -143,3 +143,27 @@ def test_wide_kernel_where_it_pays(D, B, n, n_kv, wide):
         plan = _plan(B, 16, 16, n, n_kv, D, dtype, False)
         assert (plan["kernel"] == "fa2::attn_wide_kernel") == wide, plan
         assert not wide or plan["rows"] == 256
+
+
+def _kernel(B, h_q, h_kv, n_q, n_kv, D, causal=False):
+    """The kernel of the default call (fp16: no key-norm table at these sizes), rows per workgroup."""
+    n = 1 if causal else _lib.num_splits(B, h_q, h_kv, n_q, n_kv, D, causal, 128, 0, 256)
+    plan = _plan(B, h_q, h_kv, n_q, n_kv, D, 0, causal, num_splits=n,
+                 workspace_bytes=_lib.lib().fa2_workspace_bytes(B, h_q, n_q, D, n))
+    return plan["rows"] if plan["kernel"] == WAVE_SPLIT else 0
+
+
+# Full calls on both sides of the short-key line: rows per wave-split workgroup, 0 for the general kernel
+@needs_ablate
+@pytest.mark.parametrize("shape,rows", [
+    ((6, 16, 16, 67, 150, 64), 0), ((9, 16, 8, 60, 320, 64), 0), ((3, 8, 2, 184, 370, 64), 32),
+    ((7, 16, 8, 93, 204, 64), 0), ((37, 6, 2, 60, 206, 64), 32), ((11, 12, 12, 76, 310, 64), 0),
+    ((36, 4, 4, 73, 464, 64), 64), ((9, 4, 4, 402, 239, 64), 64),
+    ((49, 8, 2, 24, 250, 128), 0), ((21, 16, 8, 45, 250, 128), 0), ((24, 20, 4, 26, 209, 128), 0),
+    ((12, 32, 8, 21, 407, 128), 0), ((14, 4, 4, 164, 467, 128), 32), ((30, 28, 4, 14, 372, 128), 64),
+    ((24, 6, 2, 68, 140, 16), 0), ((10, 28, 4, 49, 214, 16), 32),
+    ((3, 20, 4, 141, 244, 32), 0), ((8, 28, 4, 61, 302, 32), 0), ((3, 20, 4, 138, 381, 32), 32),
+    ((8, 16, 1, 1, 162, 32), 0), ((33, 6, 2, 37, 129, 32), 0), ((45, 6, 2, 27, 177, 32), 0),
+    ((41, 28, 4, 12, 179, 32), 32), ((53, 6, 2, 1, 186, 32), 32), ((8, 16, 1, 1, 194, 32), 32)])
+def test_short_keys(shape, rows):
+    assert _kernel(*shape) == rows

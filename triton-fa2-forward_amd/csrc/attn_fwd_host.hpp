@@ -155,9 +155,39 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
 //     18.5 -> 19.4, D16 15.7 -> 17.1; up to two, D32 H8 4000 x 4090 41.9 -> 33.9 but D16 N 2048 18.0 -> 18.8.
 //   * up to 128 keys (192 at head_dim 128, where tiles are small) there is little to share out:
 //     D128 H32/8 N 64 5.1 -> 6.5, N 128 6.7 -> 6.6, N 192 7.3 -> 7.3.
+//   * short keys beside a general kernel whose programs are one per CU or fewer, full, workgroups on some
+//     CUs in twos: a workgroup's few tiles do not make up for the second (general -> two on a CU).
+//     head_dim 64 rows 67 x 96 units of 150 keys 5.9 -> 6.6, 186 x 56 (112 programs) of 204 6.6 -> 6.9, but 180
+//     x 74 (222 programs) of 206 7.9 -> 7.2; 120 x 72 of 320 7.3 -> 7.7, but 736 x 12 of 370 8.0 -> 7.9, 173 x 44
+//     of 425 9.4 -> 8.2, 64 rows a workgroup 76 x 132 of 310 8.1 -> 9.5; head_dim 128 96 x 98 of 250 8.8 -> 10.7, 64 rows a workgroup 90 x 168
+//     9.7 -> 12.8, 84 x 96 of 407 11.7 -> 12.0, but 164 x 56 of 467 (the general kernel splits) 15.9 -> 12.0; groups
+//     that do not divide 128, head_dim 16 204 x 48 of 140 5.0 -> 5.7, 343 x 40 (280 programs) of 214 6.7 -> 5.7,
+//     head_dim 32 705 x 12 of 244 5.4 -> 6.3, 427 x 32 of 302 6.0 -> 6.5, 690 x 12 of 381 6.6 -> 6.4.
+//   * up to 192 keys at head_dim 32, full: two 128-key tiles, mostly masked, against three of 64 keys: 8 rows of
+//     162 keys 4.5 -> 5.1, 111 x 66 units of 129 4.8 -> 6.3; 81 x 90 in a group of 3 (270 programs) of 177 6.2 ->
+//     6.4, but 84 x 164 in a group of 7 (1148 programs) of 179 10.9 -> 6.5.
 struct KernelChoice {
   int row_waves = 0, splits = 1;
 };
+
+// The general kernel's programs in the smaller of the two GQA layouts, so that nothing chosen by them
+// depends on the packing, and the splits it is given: the smallest power of two that reaches one
+// workgroup per CU, with at least kMinSplitTiles tiles per split. (Filling the second workgroup slot of
+// each CU as well measured slower on MI355X: the fp32 partials cost more than the extra overlap gains.)
+int64_t general_programs(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int32_t block_m) {
+  const int64_t group = h_q / h_kv;
+  int64_t programs = (n_q + block_m - 1) / block_m * (batch * h_q);
+  if (block_m % group == 0)
+    programs = std::min(programs, (n_q * group + block_m - 1) / block_m * (batch * h_kv));
+  return programs;
+}
+int general_splits(int64_t programs, int64_t n_kv, int32_t bn, int cus) {
+  const int64_t tiles = (n_kv + bn - 1) / bn;
+  int s = 1;
+  while (programs * s < cus && s * 2 <= kMaxSplits && tiles / (s * 2) >= kMinSplitTiles) s *= 2;
+  return s;
+}
+
 KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64_t n_kv,
                            int32_t head_dim, bool causal, int32_t block_m, int32_t bn, int cus) {
   KernelChoice kc;
@@ -168,6 +198,7 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
   const int64_t w1 = (rows + 31) / 32 * units, w2 = (rows + 63) / 64 * units;
   const bool small = head_dim <= 32;
   const bool packs = 128 % (h_q / h_kv) == 0;  // the general kernel can pack the group
+  const int64_t programs = general_programs(batch, h_q, h_kv, n_q, block_m);
   // The splits of a launch of 32-row workgroups: doubled until one more doubling would pass one
   // workgroup per CU or leave a wave without a tile, where a wave has tiles enough for the merge
   // launch (~2 us) to pay: 7 of 32 keys x D128, or 14 where only one doubling fits. Measured (us at
@@ -195,6 +226,7 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
     kc.row_waves = 1;
     if (w1 <= cus) {
       take_splits();
+      if (head_dim == 32 && n_kv <= 192 && programs <= cus) return KernelChoice{};
       return kc;
     }
     // more 32-row workgroups than CUs (the first list above)
@@ -245,6 +277,20 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
     } else if (2 * slots >= (n_kv >= 512 ? 3 : 5) * w2) {
       kc.row_waves = 2;
     }
+  }
+  if (!causal && kc.row_waves) {  // short keys
+    bool general = false;
+    if (rows > 64 && w1 > cus && w1 <= 2 * cus && (kc.row_waves == 1 || w2 > cus)) {
+      if (head_dim == 128)
+        general = n_kv <= 448 && programs <= (w2 > cus ? 2 : 1) * cus;
+      else if (head_dim == 64)
+        general = n_kv < 336 && programs <= (kc.row_waves == 1 && n_kv > 192 ? cus / 2 : cus);
+      else
+        general = n_kv < (head_dim == 16 ? 257 : 320) && programs <= cus;
+    }
+    if (head_dim == 32 && n_kv <= 192 && kc.row_waves == 1)
+      general = general || programs <= (w1 > cus ? 2 : 1) * cus;
+    if (general) return KernelChoice{};
   }
   return kc;
 }

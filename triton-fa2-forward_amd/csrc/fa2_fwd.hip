@@ -100,21 +100,11 @@ int32_t fa2_num_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, in
   if (causal || batch <= 0 || h_q <= 0 || h_kv <= 0 || h_q % h_kv || n_q <= 0 || n_kv <= 0 ||
       block_m <= 0 || num_cus <= 0 || dim_index(head_dim) < 0)
     return 1;
-  // The grid of the smaller of the two GQA layouts, so that a packed and an unpacked launch
-  // of the same problem split the same way and stay equal bit for bit.
-  const int group = h_q / h_kv;
-  int64_t programs = ((int64_t)n_q + block_m - 1) / block_m * ((int64_t)batch * h_q);
-  if (block_m % group == 0)
-    programs = std::min(programs, ((int64_t)n_q * group + block_m - 1) / block_m * ((int64_t)batch * h_kv));
   const int bn = tile_n(block_n, head_dim);
-  const int64_t tiles = ((int64_t)n_kv + bn - 1) / bn;
-  // Split until every CU has a workgroup, with at least kMinSplitTiles tiles per split and at
-  // most kMaxSplits splits. (Filling the second workgroup slot of each CU as well measured
-  // slower on MI355X: the fp32 partial outputs cost more than the extra overlap gains.)
-  // (The wave-split kernel's few-rows launches have a count of their own, which can be larger; where
-  // it is smaller the launch itself takes fewer than it is given.)
-  int s = 1;
-  while (programs * s < num_cus && s * 2 <= kMaxSplits && tiles / (s * 2) >= kMinSplitTiles) s *= 2;
+  const int s =
+      general_splits(general_programs(batch, h_q, h_kv, n_q, block_m), n_kv, bn, num_cus);
+  // The wave-split kernel's few-rows launches have a count of their own, which can be larger; where
+  // it is smaller the launch itself takes fewer than it is given.
   const KernelChoice kc =
       kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, false, block_m, bn, num_cus);
   return kc.row_waves ? std::max(s, kc.splits) : s;
