@@ -167,3 +167,13 @@ def _kernel(B, h_q, h_kv, n_q, n_kv, D, causal=False):
     ((41, 28, 4, 12, 179, 32), 32), ((53, 6, 2, 1, 186, 32), 32), ((8, 16, 1, 1, 194, 32), 32)])
 def test_short_keys(shape, rows):
     assert _kernel(*shape) == rows
+
+
+# Causal calls of 64-row workgroups with more than one per CU, on both sides of 192 keys
+@needs_ablate
+@pytest.mark.parametrize("shape,rows", [
+    ((4, 32, 1, 165, 165, 32), 0), ((7, 16, 2, 184, 184, 32), 0), ((7, 16, 2, 193, 193, 32), 64),
+    ((10, 12, 12, 192, 192, 64), 0), ((10, 12, 12, 193, 193, 64), 64), ((10, 12, 12, 184, 184, 16), 64),
+    ((5, 16, 4, 184, 184, 32), 64), ((2, 8, 2, 184, 184, 32), 32)])
+def test_short_causal_prompts(shape, rows):
+    assert _kernel(*shape, causal=True) == rows
