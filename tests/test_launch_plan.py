@@ -174,6 +174,7 @@ def test_short_keys(shape, rows):
 @pytest.mark.parametrize("shape,rows", [
     ((4, 32, 1, 165, 165, 32), 0), ((7, 16, 2, 184, 184, 32), 0), ((7, 16, 2, 193, 193, 32), 64),
     ((10, 12, 12, 192, 192, 64), 0), ((10, 12, 12, 193, 193, 64), 64), ((10, 12, 12, 184, 184, 16), 64),
-    ((5, 16, 4, 184, 184, 32), 64), ((2, 8, 2, 184, 184, 32), 32)])
+    ((5, 16, 4, 184, 184, 32), 64), ((9, 16, 16, 191, 191, 64), 64), ((10, 20, 4, 133, 133, 32), 64),
+    ((12, 16, 8, 134, 134, 64), 0), ((2, 8, 2, 184, 184, 32), 32)])
 def test_short_causal_prompts(shape, rows):
     assert _kernel(*shape, causal=True) == rows

@@ -144,9 +144,11 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
 //     1024; its small tiles let a CU hold four workgroups) 24.0 -> 20.0, B4 (w2 2048) 34.3 -> 36.6;
 //     w2 1024 with shorter keys: D32 N 1024 14.0 -> 13.0, 512 9.1 -> 10.0; D16 N 4096 34.2 -> 29.3, 2048
 //     19.2 -> 17.2, 1024 11.1 -> 11.4 (w2 768, N 1000: 11.0 -> 10.1).
-//     64-row workgroups in twos on some CUs with short keys: D32 H32/1 B4 N 165 (w2 332) 4.9 -> 5.6, H16/2 B7
+//     64-row workgroups in twos on some CUs with short keys, beside general programs of one per CU or packed
+//     ones: D32 H32/1 B4 N 165 (w2 332) 4.9 -> 5.6, H16/2 B7
 //     184 (322) 5.0 -> 5.6, N 193-240 0.93 to 1.0 of the general kernel's time; D64 H12 B10 184 (360) 7.1 ->
-//     7.7, 193-240 0.93 to 1.01; D16 below it from 129 on.
+//     7.7, 193-240 0.93 to 1.01; but of 256 to 400 unpacked ones D64 H16 B9 191 8.7 -> 8.2, D32 H20/4 B10 133
+//     6.2 -> 5.5, and D16 below from 129 on.
 //   * full, more rows: H16 D64 N 512 9.2 -> 6.3, 1024 (w2 256) 14.4 -> 11.3, 2048 (w2 512) 27.5 ->
 //     27.2; B2 H16 D64 333 x 1500 20.7 -> 14.0; H32/8 D128 64 x 2048 B4 23.4 -> 17.2. Every row
 //     tile reads its KV head's keys again, so past some thousand keys the general kernel and its
@@ -221,7 +223,9 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
   if (causal) {  // (num_splits is 1)
     if (w1 <= cus || (w1 <= 2 * cus && n_kv >= 384))
       kc.row_waves = 1;
-    else if (w2 <= 2 * cus && n_kv >= (head_dim == 128 ? 512 : head_dim > 16 && w2 > cus ? 193 : 0))
+    else if (w2 <= 2 * cus && n_kv >= (head_dim == 128 ? 512 : 0) &&
+             !(head_dim >= 32 && n_kv <= 192 && w2 > cus &&
+               (programs <= cus || (packs && h_q > h_kv))))
       kc.row_waves = 2;
     else if (small && w2 <= 4 * cus && n_kv >= (head_dim == 16 && w2 > 3 * cus ? 1536 : 768))
       kc.row_waves = 2;
