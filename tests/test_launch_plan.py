@@ -178,3 +178,14 @@ def test_short_keys(shape, rows):
     ((12, 16, 8, 134, 134, 64), 0), ((2, 8, 2, 184, 184, 32), 32)])
 def test_short_causal_prompts(shape, rows):
     assert _kernel(*shape, causal=True) == rows
+
+
+# More than 64 rows on at most half the CUs, one range of the wave-split kernel's against the general
+# kernel's eight splits: both sides of 2560 keys, of 32 general programs and of half the CUs
+@needs_ablate
+@pytest.mark.parametrize("shape,rows", [
+    ((3, 32, 4, 31, 2560, 64), 0), ((3, 32, 4, 31, 2559, 64), 32), ((3, 32, 8, 22, 3531, 32), 0),
+    ((9, 8, 2, 36, 2984, 64), 32), ((3, 32, 8, 36, 3164, 64), 32), ((3, 16, 8, 39, 3600, 64), 32),
+    ((1, 28, 4, 103, 3388, 32), 0), ((3, 16, 8, 39, 2736, 16), 32), ((2, 8, 8, 32, 2736, 64), 32)])
+def test_long_keys_of_grids_that_leave_cus_idle(shape, rows):
+    assert _kernel(*shape) == rows

@@ -160,6 +160,10 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
 //     18.5 -> 19.4, D16 15.7 -> 17.1; up to two, D32 H8 4000 x 4090 41.9 -> 33.9 but D16 N 2048 18.0 -> 18.8.
 //   * up to 128 keys (192 at head_dim 128, where tiles are small) there is little to share out:
 //     D128 H32/8 N 64 5.1 -> 6.5, N 128 6.7 -> 6.6, N 192 7.3 -> 7.3.
+//   * full, more rows on half the CUs or fewer, keys too few for the kernel's own splits: the general kernel's
+//     eight, where they fit one per CU. D64 H16/8 B3 39 x 2736 12.9 -> 13.4, H32/4 B3 31 x 3433 14.0 -> 15.8, but 35
+//     x 2300 12.4 -> 12.2, H8/2 B9 36 x 2984 (36 programs) 15.2 -> 14.2; D32 H32/8 B3 22 x 3531 11.3 -> 12.6, H32/1 B5
+//     20 x 2262 11.0 -> 10.1.
 //   * short keys beside a general kernel whose programs are one per CU or fewer, full, workgroups on some
 //     CUs in twos: a workgroup's few tiles do not make up for the second (general -> two on a CU).
 //     head_dim 64 rows 67 x 96 units of 150 keys 5.9 -> 6.6, 186 x 56 (112 programs) of 204 6.6 -> 6.9, but 180
@@ -285,8 +289,11 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
       kc.row_waves = 2;
     }
   }
-  if (!causal && kc.row_waves) {  // short keys
-    bool general = false;
+  if (!causal && kc.row_waves) {
+    bool general = false;  // long keys: the general kernel's splits, eight or more within one per CU
+    if ((head_dim == 32 || head_dim == 64) && rows > 64 && kc.splits == 1 && 2 * w1 <= cus)
+      general = n_kv >= 2560 && 8 * programs <= cus;
+    // short keys
     if (rows > 64 && w1 > cus && w1 <= 2 * cus && (kc.row_waves == 1 || w2 > cus)) {
       if (head_dim == 128)
         general = n_kv <= 448 && programs <= (w2 > cus ? 2 : 1) * cus;
