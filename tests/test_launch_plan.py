@@ -189,3 +189,19 @@ def test_short_causal_prompts(shape, rows):
     ((1, 28, 4, 103, 3388, 32), 0), ((3, 16, 8, 39, 2736, 16), 32), ((2, 8, 8, 32, 2736, 64), 32)])
 def test_long_keys_of_grids_that_leave_cus_idle(shape, rows):
     assert _kernel(*shape) == rows
+    if rows == 0:
+        _only_with_its_splits(shape)
+
+
+def _only_with_its_splits(shape):
+    """A call that the general kernel takes for its splits: the wave-split kernel keeps it where the
+    caller allows fewer (fa2_attn_fwd: one), and the count told makes the same launch again."""
+    lib = _lib.lib()
+    B, h_q, h_kv, n_q, n_kv, D = shape
+    assert _plan(*shape, 0, False)["kernel"] == WAVE_SPLIT
+    for n in range(2, 17):
+        told = _launch_splits(*shape, n)
+        plans = [_plan(*shape, 0, False, num_splits=x,
+                       workspace_bytes=lib.fa2_workspace_bytes(B, h_q, n_q, D, x)) for x in (n, told)]
+        assert plans[0] == plans[1] and plans[0]["splits"] == told, (n, told, plans)
+        assert n >= _lib.num_splits(*shape, False, 128, 0, 256) or plans[0]["kernel"] == WAVE_SPLIT

@@ -108,7 +108,7 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
 
 // The kernel choice of a call at the default tiles: the wave-split kernel (attn_fwd_wavesplit.hpp)
 // with 32 * row_waves rows a workgroup and `splits` key ranges, or the general kernel
-// (row_waves 0; its split count is its caller's). Independent of pack, as packed and unpacked calls must agree bit for bit.
+// (row_waves 0; its split count is its caller's, at most num_splits). Independent of pack, as packed and unpacked calls must agree bit for bit.
 //
 // The wave-split kernel walks a row's keys with 4 / row_waves waves at once, which shortens a
 // launch that its longest key range bounds, but it stages K/V into LDS two or four times as often
@@ -197,8 +197,15 @@ int general_splits(int64_t programs, int64_t n_kv, int32_t bn, int cus) {
   return s;
 }
 
+// Key ranges of whole tiles that `tiles` are cut into when n are asked for: none is empty.
+int clamp_splits(int64_t tiles, int n) {
+  const int64_t per = (tiles + n - 1) / n;
+  return (int)((tiles + per - 1) / per);
+}
+
 KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64_t n_kv,
-                           int32_t head_dim, bool causal, int32_t block_m, int32_t bn, int cus) {
+                           int32_t head_dim, bool causal, int32_t block_m, int32_t bn, int cus,
+                           int num_splits) {
   KernelChoice kc;
   if (block_m != 128 || bn != default_block_n(head_dim)) return kc;
   const int64_t rows = n_q * (h_q / h_kv), units = batch * h_kv;
@@ -208,6 +215,9 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
   const bool small = head_dim <= 32;
   const bool packs = 128 % (h_q / h_kv) == 0;  // the general kernel can pack the group
   const int64_t programs = general_programs(batch, h_q, h_kv, n_q, block_m);
+  // ... and the splits it would have, which a caller that allows fewer does not give it
+  const int gs = general_splits(programs, n_kv, bn, cus);
+  const bool general_splits_ok = num_splits >= clamp_splits((n_kv + bn - 1) / bn, gs);
   // The splits of a launch of 32-row workgroups: doubled until one more doubling would pass one
   // workgroup per CU or leave a wave without a tile, where a wave has tiles enough for the merge
   // launch (~2 us) to pay: 7 of 32 keys x D128, or 14 where only one doubling fits. Measured (us at
@@ -292,7 +302,7 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
   if (!causal && kc.row_waves) {
     bool general = false;  // long keys: the general kernel's splits, eight or more within one per CU
     if ((head_dim == 32 || head_dim == 64) && rows > 64 && kc.splits == 1 && 2 * w1 <= cus)
-      general = n_kv >= 2560 && 8 * programs <= cus;
+      general = n_kv >= 2560 && 8 * programs <= cus && general_splits_ok;
     // short keys
     if (rows > 64 && w1 > cus && w1 <= 2 * cus && (kc.row_waves == 1 || w2 > cus)) {
       if (head_dim == 128)
@@ -307,12 +317,6 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
     if (general) return KernelChoice{};
   }
   return kc;
-}
-
-// Key ranges of whole tiles that `tiles` are cut into when n are asked for: none is empty.
-int clamp_splits(int64_t tiles, int n) {
-  const int64_t per = (tiles + n - 1) / n;
-  return (int)((tiles + per - 1) / per);
 }
 
 // The kernel of a launch given num_splits and the key ranges it runs: plan_launch's choice, and what
@@ -338,7 +342,7 @@ SplitChoice split_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, 
   if (n > 1 && n_kv > 0) sc.need = clamp_splits((n_kv + bn - 1) / bn, n);
   if (!general_only) {
     const KernelChoice kc =
-        kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, causal, block_m, bn, cus);
+        kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, causal, block_m, bn, cus, num_splits);
     if (kc.row_waves) {
       sc.row_waves = kc.row_waves;
       own = fa2::wave_split_block_n(head_dim, kc.row_waves, causal);

@@ -106,7 +106,7 @@ int32_t fa2_num_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, in
   // The wave-split kernel's few-rows launches have a count of their own, which can be larger; where
   // it is smaller the launch itself takes fewer than it is given.
   const KernelChoice kc =
-      kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, false, block_m, bn, num_cus);
+      kernel_choice(batch, h_q, h_kv, n_q, n_kv, head_dim, false, block_m, bn, num_cus, kMaxSplits);
   return kc.row_waves ? std::max(s, kc.splits) : s;
 }
 
