@@ -130,6 +130,13 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
 //     kernel more: D128 264 units 4 rows 2000 keys 56.6 / 62.7 / 53.9, 448 units 80.6 / 78.5 / 79.5; 264
 //     units 32 rows 206 keys 10.7 / 11.2 / 11.2; D64 264 units 2000 keys 42.0 / 32.9 / 30.2, 1000 21.3 /
 //     15.4 / 15.9; D32 336 units 206 keys 7.1 / 6.3 / 5.9, 2000 32.3 / 18.5 / 20.2.
+//   * 33 to 64 rows of packed groups at head_dim 128, where doubling the splits of the two row tiles would
+//     pass one workgroup per CU and the general kernel's one program has splits for more than that: they
+//     read the keys once. Past 544 keys a general split (2048 where few CUs idle): 16 splits H32/4 B5 12 queries
+//     of 4818 20.4 -> 18.2, B6 of 8264 32.1 -> 34.0; 8 splits H12 B3 34 x 3728 27.8 on both sides, H32/4 B10 6 x 4352
+//     28.8 -> 32.9, H12 B3 41 x 19624 80.9 -> 110.5; 4 splits H12 B6 62 x 2112 28.2 -> 26.5, 44 x 2852 33.1 -> 36.6, 33 x
+//     11666 90.8 -> 128.5; 120 units (240 workgroups) H16/8 B15 26 x 4402 61.0 -> 55.7, H32/4 B30 5 x 13079 146.5 ->
+//     152.8. At head_dim 64 no such line: -6% to +10% past 2600 keys a split, faster below.
 //   * more rows in groups that do not divide 128: the general kernel runs a program per query head,
 //     mostly of empty rows when it has few queries; full, general -> this kernel: D128 H28/4 B4 16
 //     queries of 8192 keys 50.3 -> 20.9, B1 20 of 8192 20.1 -> 15.1, B20 30 of 6000 233 -> 112, H20/4 B40
@@ -248,6 +255,10 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
     if (w1 <= cus) {
       take_splits();
       if (head_dim == 32 && n_kv <= 192 && programs <= cus) return KernelChoice{};
+      // two row tiles, long keys
+      if (head_dim == 128 && rows > 32 && packs && w1 * kc.splits < cus && programs * gs > cus &&
+          n_kv >= gs * (8 * w1 * kc.splits <= 7 * cus ? 544 : 2048) && general_splits_ok)
+        return KernelChoice{};
       return kc;
     }
     // more 32-row workgroups than CUs (the first list above)
