@@ -220,3 +220,16 @@ def test_two_row_tiles_of_long_keys(shape, rows):
     assert _kernel(*shape) == rows
     if rows == 0:
         _only_with_its_splits(shape)
+
+
+# 65 to 128 rows on one to two 32-row workgroups per CU: both sides of 1700 / 2900 keys, of 128 rows and
+# of 1.4 workgroups per CU
+@needs_ablate
+@pytest.mark.parametrize("shape,rows", [
+    ((6, 16, 16, 72, 1700, 128), 0), ((6, 16, 16, 72, 1699, 128), 32), ((10, 8, 8, 124, 2029, 128), 0),
+    ((63, 16, 2, 10, 1784, 128), 64), ((8, 8, 8, 160, 1877, 128), 32), ((12, 32, 8, 18, 2900, 64), 0),
+    ((12, 32, 8, 18, 2899, 64), 32), ((31, 32, 4, 11, 3259, 64), 64), ((3, 28, 4, 18, 1900, 128), 32)])
+def test_one_general_program_for_three_row_tiles(shape, rows):
+    assert _kernel(*shape) == rows
+    if rows == 0:
+        _only_with_its_splits(shape)

@@ -171,6 +171,10 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
 //     eight, where they fit one per CU. D64 H16/8 B3 39 x 2736 12.9 -> 13.4, H32/4 B3 31 x 3433 14.0 -> 15.8, but 35
 //     x 2300 12.4 -> 12.2, H8/2 B9 36 x 2984 (36 programs) 15.2 -> 14.2; D32 H32/8 B3 22 x 3531 11.3 -> 12.6, H32/1 B5
 //     20 x 2262 11.0 -> 10.1.
+//   * full, 65 to 128 rows of packed groups, up to 1.4 of their 32-row workgroups per CU: one general program
+//     reads the keys once for their three or four. D128 93 rows x 96 units of 1754 33.5 -> 35.1, 72 x 96 of 1993
+//     33.0 -> 38.6, but 96 x 103 of 1662 35.4 -> 35.0, 80 x 126 (1.48) of 1784 39.8 -> 37.9; D64 72 x 96 of 2930 26.5 ->
+//     27.4, 108 x 76 of 3816 30.2 -> 33.8, but 128 x 84 of 2743 25.6 -> 21.9, 88 x 124 (1.45) of 3259 34.6 both.
 //   * short keys beside a general kernel whose programs are one per CU or fewer, full, workgroups on some
 //     CUs in twos: a workgroup's few tiles do not make up for the second (general -> two on a CU).
 //     head_dim 64 rows 67 x 96 units of 150 keys 5.9 -> 6.6, 186 x 56 (112 programs) of 204 6.6 -> 6.9, but 180
@@ -311,20 +315,23 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
     }
   }
   if (!causal && kc.row_waves) {
-    bool general = false;  // long keys: the general kernel's splits, eight or more within one per CU
+    bool general = false;
+    // long keys: the general kernel's splits
     if ((head_dim == 32 || head_dim == 64) && rows > 64 && kc.splits == 1 && 2 * w1 <= cus)
-      general = n_kv >= 2560 && 8 * programs <= cus && general_splits_ok;
+      general |= n_kv >= 2560 && 8 * programs <= cus && general_splits_ok;
+    if (head_dim >= 64 && rows > 64 && rows <= 128 && packs && w1 > cus && 5 * w1 <= 7 * cus)
+      general |= n_kv >= (head_dim == 64 ? 2900 : 1700) && general_splits_ok;
     // short keys
     if (rows > 64 && w1 > cus && w1 <= 2 * cus && (kc.row_waves == 1 || w2 > cus)) {
       if (head_dim == 128)
-        general = n_kv <= 448 && programs <= (w2 > cus ? 2 : 1) * cus;
+        general |= n_kv <= 448 && programs <= (w2 > cus ? 2 : 1) * cus;
       else if (head_dim == 64)
-        general = n_kv < 336 && programs <= (kc.row_waves == 1 && n_kv > 192 ? cus / 2 : cus);
+        general |= n_kv < 336 && programs <= (kc.row_waves == 1 && n_kv > 192 ? cus / 2 : cus);
       else
-        general = n_kv < (head_dim == 16 ? 257 : 320) && programs <= cus;
+        general |= n_kv < (head_dim == 16 ? 257 : 320) && programs <= cus;
     }
     if (head_dim == 32 && n_kv <= 192 && kc.row_waves == 1)
-      general = general || programs <= (w1 > cus ? 2 : 1) * cus;
+      general |= programs <= (w1 > cus ? 2 : 1) * cus;
     if (general) return KernelChoice{};
   }
   return kc;
