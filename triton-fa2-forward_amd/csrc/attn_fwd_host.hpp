@@ -107,85 +107,94 @@ bool key_table_pays(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, int64
 }
 
 // The kernel choice of a call at the default tiles: the wave-split kernel (attn_fwd_wavesplit.hpp)
-// with 32 * row_waves rows a workgroup and `splits` key ranges, or the general kernel
-// (row_waves 0; its split count is its caller's, at most num_splits). Independent of pack, as packed and unpacked calls must agree bit for bit.
-//
-// The wave-split kernel walks a row's keys with 4 / row_waves waves at once, which shortens a
-// launch that its longest key range bounds, but it stages K/V into LDS two or four times as often
-// per row, so a grid that fills the GPU belongs to the general kernel. Where the line lies was
-// measured on MI355X (us per launch in a graph, general kernel -> this one; w1 and w2 are the
-// workgroups at 32 and 64 rows; 256 CUs hold two of them each):
+// with 32 * row_waves rows a workgroup and `splits` key ranges, or the general kernel (row_waves 0;
+// its split count is its caller's, at most num_splits). Independent of pack, as packed and unpacked
+// calls must agree bit for bit. The wave-split kernel walks a row's keys with 4 / row_waves waves
+// at once, which shortens a launch that its longest key range bounds, but it stages K/V into LDS
+// two or four times as often per row, so a grid that fills the GPU belongs to the general kernel.
+// Where the line lies was measured on MI355X (us per launch in a graph, general kernel -> this one;
+// w1 and w2 are the workgroups at 32 and 64 rows; 256 CUs hold two of them each):
 //   * few rows (at most 64 per KV head, not causal), bound by reading K/V: bf16 H32/8 D128 one
-//     query of 32000 keys 50.5 -> 32.4, of 1000 10.1 -> 7.9, B16 4096 keys 59.9 -> 49.4, B16 with 16
-//     queries 62.2 -> 53.4, H28/4 D64 B8 5712 keys 53.4 -> 15.1 (the general kernel cannot pack a
-//     group of 7).
-//   * few rows in more 32-row workgroups than CUs. 33 to 64 rows: two row tiles read every key twice,
-//     so 64 rows a workgroup, or, where the general kernel packs the group, its one program (general /
-//     32 / 64 rows a workgroup; units are KV heads): D128 336 units 64 rows 206 keys 12.8 / 16.0 / 13.7,
-//     2000 67.9 / 74.5 / 68.9; 160 units 48 rows 206 keys 9.0 / 10.3 / 8.7, 700 19.6 / 16.4 / 14.8, 4000
-//     (the general kernel splits) 70.4 / 83.5 / 81.2; 248 units 64 rows 700 keys 31.1 / 21.0 / 20.4. D64
-//     336 units 64 rows 1000 keys 24.1 / 21.2 / 19.7, 136 units 36 rows 206 keys 7.0 / 6.9 / 6.1, but 600
-//     units (one round of the general kernel) 700 keys 28.0 / 29.9 / 29.3. D32 336 units 64 rows 2000
-//     keys 32.6 / 22.4 / 21.2, but 248 units of 4000 keys 44.1 / 28.7 / 32.6. Up to 32 rows: a last round that few workgroups reach costs the 32-row
-//     kernel more: D128 264 units 4 rows 2000 keys 56.6 / 62.7 / 53.9, 448 units 80.6 / 78.5 / 79.5; 264
-//     units 32 rows 206 keys 10.7 / 11.2 / 11.2; D64 264 units 2000 keys 42.0 / 32.9 / 30.2, 1000 21.3 /
-//     15.4 / 15.9; D32 336 units 206 keys 7.1 / 6.3 / 5.9, 2000 32.3 / 18.5 / 20.2.
-//   * 33 to 64 rows of packed groups at head_dim 128, where doubling the splits of the two row tiles would
-//     pass one workgroup per CU and the general kernel's one program has splits for more than that: they
-//     read the keys once. Past 544 keys a general split (2048 where few CUs idle): 16 splits H32/4 B5 12 queries
-//     of 4818 20.4 -> 18.2, B6 of 8264 32.1 -> 34.0; 8 splits H12 B3 34 x 3728 27.8 on both sides, H32/4 B10 6 x 4352
-//     28.8 -> 32.9, H12 B3 41 x 19624 80.9 -> 110.5; 4 splits H12 B6 62 x 2112 28.2 -> 26.5, 44 x 2852 33.1 -> 36.6, 33 x
-//     11666 90.8 -> 128.5; 120 units (240 workgroups) H16/8 B15 26 x 4402 61.0 -> 55.7, H32/4 B30 5 x 13079 146.5 ->
-//     152.8. At head_dim 64 no such line: -6% to +10% past 2600 keys a split, faster below.
+//     query of 32000 keys 50.5 -> 32.4, of 1000 10.1 -> 7.9, B16 4096 keys 59.9 -> 49.4, B16 with
+//     16 queries 62.2 -> 53.4, H28/4 D64 B8 5712 keys 53.4 -> 15.1 (the general kernel cannot pack
+//     a group of 7).
+//   * few rows in more 32-row workgroups than CUs. 33 to 64 rows: two row tiles read every key
+//     twice, so 64 rows a workgroup, or, where the general kernel packs the group, its one program
+//     (general / 32 / 64 rows a workgroup; units are KV heads): D128 336 units 64 rows 206 keys
+//     12.8 / 16.0 / 13.7, 2000 67.9 / 74.5 / 68.9; 160 units 48 rows 206 keys 9.0 / 10.3 / 8.7, 700
+//     19.6 / 16.4 / 14.8, 4000 (the general kernel splits) 70.4 / 83.5 / 81.2; 248 units 64 rows
+//     700 keys 31.1 / 21.0 / 20.4. D64 336 units 64 rows 1000 keys 24.1 / 21.2 / 19.7, 136 units 36
+//     rows 206 keys 7.0 / 6.9 / 6.1, but 600 units (one round of the general kernel) 700 keys 28.0
+//     / 29.9 / 29.3. D32 336 units 64 rows 2000 keys 32.6 / 22.4 / 21.2, but 248 units of 4000 keys
+//     44.1 / 28.7 / 32.6. Up to 32 rows: a last round that few workgroups reach costs the 32-row
+//     kernel more: D128 264 units 4 rows 2000 keys 56.6 / 62.7 / 53.9, 448 units 80.6 / 78.5 /
+//     79.5; 264 units 32 rows 206 keys 10.7 / 11.2 / 11.2; D64 264 units 2000 keys 42.0 / 32.9 /
+//     30.2, 1000 21.3 / 15.4 / 15.9; D32 336 units 206 keys 7.1 / 6.3 / 5.9, 2000 32.3 / 18.5 /
+//     20.2.
+//   * 33 to 64 rows of packed groups at head_dim 128, where doubling the splits of the two row
+//     tiles would pass one workgroup per CU and the general kernel's one program has splits for
+//     more than that: they read the keys once. Past 544 keys a general split (660 of four, 2048
+//     where few CUs idle): 16 splits H32/4 B5 12 queries of 4818 20.4 -> 18.2, B6 of 8264 32.1 ->
+//     34.0; 8 splits H12 B3 34 x 3728 27.8 on both sides, H32/4 B10 6 x 4352 28.8 -> 32.9, H12 B3
+//     41 x 19624 80.9 -> 110.5; 4 splits H8 B12 59 x 2467 35.0 -> 31.9, H12 B6 44 x 2852 33.1 ->
+//     36.6, 33 x 11666 90.8 -> 128.5; 120 units (240 workgroups) H16/8 B15 26 x 4402 61.0 -> 55.7,
+//     H32/4 B30 5 x 13079 146.5 -> 152.8. At head_dim 64 no such line: -6% to +10% past 2600 keys a
+//     split, faster below.
 //   * more rows in groups that do not divide 128: the general kernel runs a program per query head,
 //     mostly of empty rows when it has few queries; full, general -> this kernel: D128 H28/4 B4 16
-//     queries of 8192 keys 50.3 -> 20.9, B1 20 of 8192 20.1 -> 15.1, B20 30 of 6000 233 -> 112, H20/4 B40
-//     16 of 1000 50.0 -> 26.0; D64 H28/4 B4 16 of 8192 39.5 -> 14.4. With long keys on grids of more than
-//     half the CUs 64 rows a workgroup and splits beat 32: B8 40 of 8000 99.4 / 89.6 / 75.0, H20/4 B12 64
-//     of 20000 277 / 293 / 200. It takes 1.5 times the rows' own slots to be worth it (2.5 below 512
-//     keys): H28/4 B1 200 of 8000 (1.27) 39.9 -> 45.2, B30 60 of 300 (2.0) 23.3 -> 24.8.
-//   * causal, one round of workgroups (D128 H8/2): N 512 12.5 -> 8.5, 1024 20.8 -> 11.5, 2048
-//     37.5 -> 20.9, 4096 (w2 512) 69.7 -> 55.1; H32/8 N 256 8.9 -> 7.4, 512 13.0 -> 10.7, 1024
-//     (w2 512) 22.7 -> 20.3, but 2048 (w2 1024) 45.8 -> 50.5. D64 H16 N 256 7.7 -> 5.7, 1024 16.0
-//     -> 9.3, 2048 (w2 512) 28.4 -> 20.7; B4 1024 (w2 1024) 19.9 -> 23.1. D32 H16 B2 N 2048 (w2
-//     1024; its small tiles let a CU hold four workgroups) 24.0 -> 20.0, B4 (w2 2048) 34.3 -> 36.6;
-//     w2 1024 with shorter keys: D32 N 1024 14.0 -> 13.0, 512 9.1 -> 10.0; D16 N 4096 34.2 -> 29.3, 2048
-//     19.2 -> 17.2, 1024 11.1 -> 11.4 (w2 768, N 1000: 11.0 -> 10.1).
-//     64-row workgroups in twos on some CUs with short keys, beside general programs of one per CU or packed
-//     ones: D32 H32/1 B4 N 165 (w2 332) 4.9 -> 5.6, H16/2 B7
-//     184 (322) 5.0 -> 5.6, N 193-240 0.93 to 1.0 of the general kernel's time; D64 H12 B10 184 (360) 7.1 ->
-//     7.7, 193-240 0.93 to 1.01; but of 256 to 400 unpacked ones D64 H16 B9 191 8.7 -> 8.2, D32 H20/4 B10 133
-//     6.2 -> 5.5, and D16 below from 129 on.
+//     queries of 8192 keys 50.3 -> 20.9, B1 20 of 8192 20.1 -> 15.1, B20 30 of 6000 233 -> 112,
+//     H20/4 B40 16 of 1000 50.0 -> 26.0; D64 H28/4 B4 16 of 8192 39.5 -> 14.4. With long keys on
+//     grids of more than half the CUs 64 rows a workgroup and splits beat 32: B8 40 of 8000 99.4 /
+//     89.6 / 75.0, H20/4 B12 64 of 20000 277 / 293 / 200. It takes 1.5 times the rows' own slots to
+//     be worth it (2.5 below 512 keys): H28/4 B1 200 of 8000 (1.27) 39.9 -> 45.2, B30 60 of 300
+//     (2.0) 23.3 -> 24.8.
+//   * causal, one round of workgroups (D128 H8/2): N 512 12.5 -> 8.5, 1024 20.8 -> 11.5, 2048 37.5
+//     -> 20.9, 4096 (w2 512) 69.7 -> 55.1; H32/8 N 256 8.9 -> 7.4, 512 13.0 -> 10.7, 1024 (w2 512)
+//     22.7 -> 20.3, but 2048 (w2 1024) 45.8 -> 50.5. D64 H16 N 256 7.7 -> 5.7, 1024 16.0 -> 9.3,
+//     2048 (w2 512) 28.4 -> 20.7; B4 1024 (w2 1024) 19.9 -> 23.1. D32 H16 B2 N 2048 (w2 1024; its
+//     small tiles let a CU hold four workgroups) 24.0 -> 20.0, B4 (w2 2048) 34.3 -> 36.6; w2 1024
+//     with shorter keys: D32 N 1024 14.0 -> 13.0, 512 9.1 -> 10.0; D16 N 4096 34.2 -> 29.3, 2048
+//     19.2 -> 17.2, 1024 11.1 -> 11.4 (w2 768, N 1000: 11.0 -> 10.1). 64-row workgroups in twos on
+//     some CUs with short keys, beside general programs of one per CU or packed ones: D32 H32/1 B4
+//     N 165 (w2 332) 4.9 -> 5.6, H16/2 B7 184 (322) 5.0 -> 5.6, N 193-240 0.93 to 1.0 of the
+//     general kernel's time; D64 H12 B10 184 (360) 7.1 -> 7.7, 193-240 0.93 to 1.01; but of 256 to
+//     400 unpacked ones D64 H16 B9 191 8.7 -> 8.2, D32 H20/4 B10 133 6.2 -> 5.5, and D16 below from
+//     129 on.
 //   * full, more rows: H16 D64 N 512 9.2 -> 6.3, 1024 (w2 256) 14.4 -> 11.3, 2048 (w2 512) 27.5 ->
 //     27.2; B2 H16 D64 333 x 1500 20.7 -> 14.0; H32/8 D128 64 x 2048 B4 23.4 -> 17.2. Every row
 //     tile reads its KV head's keys again, so past some thousand keys the general kernel and its
 //     split are better: H32/8 D128 128 x 4096 24.6 -> 26.3, D64 H16 256 x 8192 23.0 -> 29.8.
 //   * full at head_dim 16 and 32 on w2 of 2 to 3 workgroups per CU: the general kernel's 128-row
 //     programs leave CUs with one beside CUs with two, and 64 rows spread more evenly, at any key
-//     count: D32 H8 4160 x 512 10.4 -> 9.7, x 4090 58.6 -> 42.6, x 16000 217.7 -> 148.2, 6144 x 16000
-//     217.4 -> 160.3; D16 4160 x 700 12.7 -> 11.4, x 16000 169.4 -> 150.9. Past three, D32 H16 4096 x 1000
-//     18.5 -> 19.4, D16 15.7 -> 17.1; up to two, D32 H8 4000 x 4090 41.9 -> 33.9 but D16 N 2048 18.0 -> 18.8.
+//     count: D32 H8 4160 x 512 10.4 -> 9.7, x 4090 58.6 -> 42.6, x 16000 217.7 -> 148.2, 6144 x
+//     16000 217.4 -> 160.3; D16 4160 x 700 12.7 -> 11.4, x 16000 169.4 -> 150.9. Past three, D32
+//     H16 4096 x 1000 18.5 -> 19.4, D16 15.7 -> 17.1; up to two, D32 H8 4000 x 4090 41.9 -> 33.9
+//     but D16 N 2048 18.0 -> 18.8.
 //   * up to 128 keys (192 at head_dim 128, where tiles are small) there is little to share out:
 //     D128 H32/8 N 64 5.1 -> 6.5, N 128 6.7 -> 6.6, N 192 7.3 -> 7.3.
-//   * full, more rows on half the CUs or fewer, keys too few for the kernel's own splits: the general kernel's
-//     eight, where they fit one per CU. D64 H16/8 B3 39 x 2736 12.9 -> 13.4, H32/4 B3 31 x 3433 14.0 -> 15.8, but 35
-//     x 2300 12.4 -> 12.2, H8/2 B9 36 x 2984 (36 programs) 15.2 -> 14.2; D32 H32/8 B3 22 x 3531 11.3 -> 12.6, H32/1 B5
-//     20 x 2262 11.0 -> 10.1.
-//   * full, 65 to 128 rows of packed groups, up to 1.4 of their 32-row workgroups per CU: one general program
-//     reads the keys once for their three or four. D128 93 rows x 96 units of 1754 33.5 -> 35.1, 72 x 96 of 1993
-//     33.0 -> 38.6, but 96 x 103 of 1662 35.4 -> 35.0, 80 x 126 (1.48) of 1784 39.8 -> 37.9; D64 72 x 96 of 2930 26.5 ->
-//     27.4, 108 x 76 of 3816 30.2 -> 33.8, but 128 x 84 of 2743 25.6 -> 21.9, 88 x 124 (1.45) of 3259 34.6 both.
-//   * short keys beside a general kernel whose programs are one per CU or fewer, full, workgroups on some
-//     CUs in twos: a workgroup's few tiles do not make up for the second (general -> two on a CU).
-//     head_dim 64 rows 67 x 96 units of 150 keys 5.9 -> 6.6, 186 x 56 (112 programs) of 204 6.6 -> 6.9, but 180
-//     x 74 (222 programs) of 206 7.9 -> 7.2; 120 x 72 of 320 7.3 -> 7.7, but 736 x 12 of 370 8.0 -> 7.9, 173 x 44
-//     of 425 9.4 -> 8.2, 64 rows a workgroup 76 x 132 of 310 8.1 -> 9.5; head_dim 128 96 x 98 of 250 8.8 -> 10.7, 64 rows a workgroup 90 x 168
-//     9.7 -> 12.8, 84 x 96 of 407 11.7 -> 12.0, but 164 x 56 of 467 (the general kernel splits) 15.9 -> 12.0; groups
-//     that do not divide 128, head_dim 16 204 x 48 of 140 5.0 -> 5.7, 343 x 40 (280 programs) of 214 6.7 -> 5.7,
-//     head_dim 32 705 x 12 of 244 5.4 -> 6.3, 427 x 32 of 302 6.0 -> 6.5, 690 x 12 of 381 6.6 -> 6.4.
-//   * up to 192 keys at head_dim 32, full: two 128-key tiles, mostly masked, against three of 64 keys: 8 rows of
-//     162 keys 4.5 -> 5.1, 111 x 66 units of 129 4.8 -> 6.3; 81 x 90 in a group of 3 (270 programs) of 177 6.2 ->
-//     6.4, but 84 x 164 in a group of 7 (1148 programs) of 179 10.9 -> 6.5.
+//   * full, more rows on half the CUs or fewer, keys too few for the kernel's own splits: the
+//     general kernel's eight, where they fit one per CU. D64 H16/8 B3 39 x 2736 12.9 -> 13.4, H32/4
+//     B3 31 x 3433 14.0 -> 15.8, but 35 x 2300 12.4 -> 12.2, H8/2 B9 36 x 2984 (36 programs) 15.2
+//     -> 14.2; D32 H32/8 B3 22 x 3531 11.3 -> 12.6, H32/1 B5 20 x 2262 11.0 -> 10.1.
+//   * full, 65 to 128 rows of packed groups, up to 1.4 of their 32-row workgroups per CU: one
+//     general program reads the keys once for their three or four. D128 93 rows x 96 units of 1754
+//     33.5 -> 35.1, 72 x 96 of 1993 33.0 -> 38.6, but 96 x 103 of 1662 35.4 -> 35.0, 80 x 126
+//     (1.48) of 1784 39.8 -> 37.9; D64 72 x 96 of 2930 26.5 -> 27.4, 108 x 76 of 3816 30.2 -> 33.8,
+//     but 128 x 84 of 2743 25.6 -> 21.9, 88 x 124 (1.45) of 3259 34.6 both.
+//   * short keys beside a general kernel whose programs are one per CU or fewer, full, workgroups
+//     on some CUs in twos: a workgroup's few tiles do not make up for the second (general -> two on
+//     a CU). head_dim 64 rows 67 x 96 units of 150 keys 5.9 -> 6.6, 186 x 56 (112 programs) of 204
+//     6.6 -> 6.9, but 180 x 74 (222 programs) of 206 7.9 -> 7.2; 120 x 72 of 320 7.3 -> 7.7, but
+//     736 x 12 of 370 8.0 -> 7.9, 173 x 44 of 425 9.4 -> 8.2, 64 rows a workgroup 76 x 132 of 310
+//     8.1 -> 9.5; head_dim 128 96 x 98 of 250 8.8 -> 10.7, 64 rows a workgroup 90 x 168 9.7 ->
+//     12.8, 84 x 96 of 407 11.7 -> 12.0, but 164 x 56 of 467 (the general kernel splits) 15.9 ->
+//     12.0; groups that do not divide 128, head_dim 16 204 x 48 of 140 5.0 -> 5.7, 343 x 40 (280
+//     programs) of 214 6.7 -> 5.7, head_dim 32 705 x 12 of 244 5.4 -> 6.3, 427 x 32 of 302 6.0 ->
+//     6.5, 690 x 12 of 381 6.6 -> 6.4.
+//   * up to 192 keys at head_dim 32, full: two 128-key tiles, mostly masked, against three of 64
+//     keys: 8 rows of 162 keys 4.5 -> 5.1, 111 x 66 units of 129 4.8 -> 6.3; 81 x 90 in a group of
+//     3 (270 programs) of 177 6.2 -> 6.4, but 84 x 164 in a group of 7 (1148 programs) of 179 10.9
+//     -> 6.5.
 struct KernelChoice {
   int row_waves = 0, splits = 1;
 };
@@ -261,7 +270,7 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
       if (head_dim == 32 && n_kv <= 192 && programs <= cus) return KernelChoice{};
       // two row tiles, long keys
       if (head_dim == 128 && rows > 32 && packs && w1 * kc.splits < cus && programs * gs > cus &&
-          n_kv >= gs * (8 * w1 * kc.splits <= 7 * cus ? 544 : 2048) && general_splits_ok)
+          n_kv >= gs * (8 * w1 * kc.splits > 7 * cus ? 2048 : gs > 4 ? 544 : 660) && general_splits_ok)
         return KernelChoice{};
       return kc;
     }
