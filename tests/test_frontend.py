@@ -587,6 +587,25 @@ def test_default_instances_keep_the_occupancy_the_design_counts_on():
 
 
 @needs_lib
+def test_native_call_is_used_only_with_the_torch_it_was_built_for(monkeypatch):
+    """fa2/_torch_call.so reads tensors by their C++ layout, so a torch or Python other than the one it
+    was compiled against must not get it, even where every symbol resolves."""
+    from fa2 import _torch_call
+
+    assert _torch_call.built_for == _lib.build_id()
+    assert _lib._load_fast_call() is _torch_call.call
+    with monkeypatch.context() as m:
+        m.setattr(torch, "__version__", "2.99.0")
+        assert _lib._load_fast_call() is None
+    with monkeypatch.context() as m:
+        m.setattr(torch.version, "git_version", "0" * 40)
+        assert _lib._load_fast_call() is None
+    with monkeypatch.context() as m:
+        m.setattr("sys.version_info", (3, 99, 0))
+        assert _lib._load_fast_call() is None
+
+
+@needs_lib
 def test_fa2_installs_as_a_package(tmp_path):
     """`pip install .` puts the drop-in under its reference import name with the built library
     inside, so `from fa2.kernel import

@@ -176,7 +176,7 @@ def build(jobs=8, verbose=False):
                "-o", os.path.join(OBJ_DIR, "mfma_ceiling.o")]
     torch_obj = os.path.join(OBJ_DIR, "fa2_torch.o")
     torch_call = ["g++", "-std=c++20", "-O2", "-fPIC", "-fvisibility=hidden", "-Wall",
-                  "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", "-I", INCLUDE,
+                  "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", f'-DFA2_BUILT_FOR="{torch_build_id()}"', "-I", INCLUDE,
                   *(f for p in torch_paths()[0] for f in ("-isystem", p)), "-c",
                   os.path.join(CSRC, "fa2_torch.cpp"), "-o", torch_obj]
     everything = units + shared + [api, scratch] + ablate_units + [ablate_api, ablate_split, ceiling, torch_call]
@@ -208,6 +208,16 @@ def build(jobs=8, verbose=False):
     os.replace(TORCH_CALL_PATH + ".tmp", TORCH_CALL_PATH)
     build_capi_check(verbose)
     return LIB_PATH
+
+
+def torch_build_id():
+    """fa2/_lib.py's build_id() of the installed torch and this Python, without importing torch."""
+    import importlib.util
+    import runpy
+
+    torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    v = runpy.run_path(os.path.join(torch_dir, "version.py"))
+    return "torch {} {} python {}.{}".format(v["__version__"], v["git_version"], *sys.version_info[:2])
 
 
 def torch_paths():

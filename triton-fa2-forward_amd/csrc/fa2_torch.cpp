@@ -201,4 +201,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_torch_call", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__torch_call() { return PyModule_Create(&module); }
+// built_for: fa2/_lib.py's build_id() of the torch and Python compiled against (csrc/build.py); another
+// one does not use this module.
+PyMODINIT_FUNC PyInit__torch_call() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_for", FA2_BUILT_FOR) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -8,6 +8,7 @@ torch hands out.
 
 import ctypes
 import os
+import sys
 
 import torch  # noqa: F401  (must be loaded before the HIP library, see above)
 
@@ -60,13 +61,25 @@ def lib():
     return _LIB
 
 
-# The native common call of attention() (csrc/fa2_torch.cpp), built beside the library against this
-# torch; None where it is missing or was built for another torch: attention() then makes every
-# call itself, through ctypes.
-try:
-    from ._torch_call import call as fast_call
-except ImportError:
-    fast_call = None
+def build_id():
+    """The torch and the Python that the native call must have been built for: it reads tensors by
+    their C++ layout, which another build of either can change without a missing symbol."""
+    return "torch {} {} python {}.{}".format(torch.__version__, torch.version.git_version,
+                                             *sys.version_info[:2])
+
+
+def _load_fast_call():
+    """The native common call of attention() (csrc/fa2_torch.cpp), built beside the library; None where
+    it is missing or was built for another torch or Python: attention() then makes every call itself,
+    through ctypes."""
+    try:
+        from . import _torch_call
+    except ImportError:
+        return None
+    return _torch_call.call if getattr(_torch_call, "built_for", None) == build_id() else None
+
+
+fast_call = _load_fast_call()
 
 
 def last_error():
