@@ -568,6 +568,44 @@ def test_build_records_the_resources_of_every_product_instance():
 
 
 @needs_lib
+def test_record_and_occupancy_of_the_wave_split_and_wide_kernels():
+    """Every instance that a default call runs is in the record, without VGPR spills, and as many
+    workgroups fit a CU as the rules count on (attn_fwd_host.hpp): two of the wave-split kernel's,
+    which split_program pairs, four of its 64-row causal ones at head_dim 16 and 32, and two and three of
+    the wide kernel's at head_dim 64 and 32."""
+    import sweep
+
+    res = sweep.load_resources()
+    seen = {}
+    for r in res.values():
+        seen.setdefault(r["kernel"], []).append(r)
+    assert len(seen["attn_wave_split_kernel"]) == 2 * 4 * 2 * 2 and len(seen["attn_wide_kernel"]) == 2 * 2 * 2
+    for r in seen["attn_wave_split_kernel"]:
+        fit = 4 if r["block_m"] == 64 and r["causal"] and r["head_dim"] <= 32 else 2
+        assert r["waves_per_simd"] >= fit and r["lds_bytes"] * fit <= 160 * 1024 and r["vgpr_spills"] == 0, r
+    for r in seen["attn_wide_kernel"]:
+        fit = 3 if r["head_dim"] == 32 else 2
+        assert r["waves_per_simd"] >= fit and r["lds_bytes"] * fit <= 160 * 1024 and r["vgpr_spills"] == 0, r
+
+
+@needs_lib
+@needs_ablate
+def test_sweep_names_the_kernel_a_call_runs():
+    import sweep
+    from ablation import launch_plan
+
+    res = sweep.load_resources()
+    for args, kw, kernel in (((1, 4, 4, 256, 256, 64, 0, True), {}, "attn_wave_split_kernel"),
+                             ((8, 16, 16, 1024, 1024, 64, 1, False), {}, "attn_wide_kernel"),
+                             ((2, 16, 16, 16384, 16384, 64, 0, False), {"workspace_bytes": 1 << 20}, "attn_wide_kernel"),
+                             ((4, 16, 16, 4096, 4096, 128, 1, True), {}, "attn_fwd_kernel"),
+                             ((1, 4, 4, 256, 256, 64, 0, True), {"block_m": 64}, "attn_fwd_kernel")):
+        plan = launch_plan(*args, **kw)
+        r = res[sweep.plan_instance(plan, args[6], args[5], kw.get("block_m", 128), args[7])]
+        assert r["kernel"] == kernel and r["block_n"] == plan["keys"] and r["block_m"] == plan["rows"], (r, plan)
+
+
+@needs_lib
 def test_default_instances_keep_the_occupancy_the_design_counts_on():
     """The compiler's report of the default instances: two waves per SIMD and no VGPR spills at
     head_dim 128 (C2, C3, C5; with and without the key-norm table), three waves per SIMD for the

@@ -88,26 +88,39 @@ _REMARK = re.compile(r"remark:\s+(Function Name|TotalSGPRs|VGPRs|AGPRs|ScratchSi
 _FIELDS = {"TotalSGPRs": "sgprs", "VGPRs": "vgprs", "AGPRs": "agprs",
            "ScratchSize [bytes/lane]": "scratch_bytes_per_lane", "Occupancy [waves/SIMD]": "waves_per_simd",
            "SGPRs Spill": "sgpr_spills", "VGPRs Spill": "vgpr_spills", "LDS Size [bytes/block]": "lds_bytes"}
-_KERNEL = re.compile(r"^_ZN3fa215attn_fwd_kernelILi(\d)ELi(\d+)ELi(\d)ELi(\d+)ELb([01])ELi(\d+)EEEvNS_6ParamsE$")
+# the three attention kernels' template arguments in their mangled names
+_KERNELS = {
+    "attn_fwd_kernel": re.compile(r"^_ZN3fa215attn_fwd_kernelILi(\d)ELi(\d+)ELi(\d)ELi(\d+)ELb([01])ELi(\d+)EEEv"),
+    "attn_wave_split_kernel": re.compile(
+        r"^_ZN3fa222attn_wave_split_kernelILi(\d)ELi(\d+)ELi(\d)ELi(\d+)ELb([01])ELi(\d+)EEEv"),
+    "attn_wide_kernel": re.compile(r"^_ZN3fa216attn_wide_kernelILi(\d)ELi(\d+)ELb([01])EEEv"),
+}
 
 
 def parse_resources(stderr):
-    """kernel-resource-usage remarks -> {mangled name: {field: int}} for the forward kernel."""
+    """kernel-resource-usage remarks -> {mangled name: {field: int}} for the attention kernels."""
     out, cur = {}, None
     for m in _REMARK.finditer(stderr):
         key, val = m.group(1), m.group(2)
         if key == "Function Name":
-            cur = out.setdefault(val, {}) if _KERNEL.match(val) else None
+            cur = out.setdefault(val, {}) if any(k.match(val) for k in _KERNELS.values()) else None
         elif cur is not None:
             cur[_FIELDS[key]] = int(val)
     return out
 
 
 def describe_instance(name):
-    """attn_fwd_kernel<DT, D, NW, BN, CAUSAL, VARIANT> template arguments of a mangled name."""
-    m = _KERNEL.match(name)
-    dt, d, nw, bn, causal, variant = (int(x) for x in m.groups())
-    return {"dtype": ("fp16", "bf16")[dt], "head_dim": d, "waves": nw, "block_m": 32 * nw,
+    """The template arguments of a mangled name: attn_fwd_kernel<DT, D, NW, BN, CAUSAL, VARIANT>,
+    attn_wave_split_kernel<DT, D, GW, BN, CAUSAL, VARIANT> or attn_wide_kernel<DT, D, KB>. block_m is the
+    rows per workgroup; variant 4 uses the key-norm table."""
+    kernel, m = next((k, r.match(name)) for k, r in _KERNELS.items() if r.match(name))
+    dt, d, *rest = (int(x) for x in m.groups())
+    if kernel == "attn_wide_kernel":
+        waves, rows, bn, causal, variant = 4, 256, 64, 0, 4 * rest[0]
+    else:
+        nw, bn, causal, variant = rest
+        waves, rows = (nw, 32 * nw) if kernel == "attn_fwd_kernel" else (4, 32 * nw)
+    return {"kernel": kernel, "dtype": ("fp16", "bf16")[dt], "head_dim": d, "waves": waves, "block_m": rows,
             "block_n": bn, "causal": bool(causal), "variant": variant}
 
 
@@ -160,8 +173,9 @@ def build(jobs=8, verbose=False):
             ablate_units.append([cc, *common_flags(), f"-DFA2_DT={dt}", f"-DFA2_D={d}", "-c",
                                  os.path.join(CSRC, "attn_fwd_ablate_inst.hip"), "-o", obj])
     shared = []
-    for name in ("attn_fwd_combine", "attn_fwd_wavesplit", "attn_key_norm"):
-        shared.append([cc, *common_flags(), "-c", os.path.join(CSRC, name + ".hip"),
+    for name in ("attn_fwd_wavesplit", "attn_fwd_combine", "attn_key_norm"):
+        remarks = ["-Rpass-analysis=kernel-resource-usage"] if name == "attn_fwd_wavesplit" else []
+        shared.append([cc, *common_flags(), *remarks, "-c", os.path.join(CSRC, name + ".hip"),
                        "-o", os.path.join(OBJ_DIR, name + ".o")])
     api = [cc, *common_flags(), "-c", os.path.join(CSRC, "fa2_fwd.hip"),
            "-o", os.path.join(OBJ_DIR, "fa2_fwd.o")]
@@ -184,7 +198,7 @@ def build(jobs=8, verbose=False):
         errs = list(ex.map(lambda cmd: _run(cmd, verbose), everything))
 
     resources = {}
-    for err in errs[:len(units)]:
+    for err in errs[:len(units) + 1]:  # ... and the wave-split unit, the first shared one
         for name, fields in parse_resources(err).items():
             resources[name] = {**describe_instance(name), **fields}
     with open(RESOURCES_PATH + ".tmp", "w") as f:

@@ -39,9 +39,20 @@ def load_resources():
         return {}
 
 
+def plan_instance(plan, dtype_code, head_dim, block_m, causal):
+    """Mangled name of the instance a launch plan (ablation.launch_plan) runs."""
+    if plan["kernel"] == "fa2::attn_wave_split_kernel":
+        return (f"_ZN3fa222attn_wave_split_kernelILi{dtype_code}ELi{head_dim}ELi{plan['rows'] // 32}"
+                f"ELi{plan['keys']}ELb{int(bool(causal))}ELi0EEEvNS_6ParamsE")
+    if plan["kernel"] == "fa2::attn_wide_kernel":
+        return (f"_ZN3fa216attn_wide_kernelILi{dtype_code}ELi{head_dim}ELb{int(plan['key_table'])}"
+                "EEEvNS_6ParamsE")
+    return instance_name(dtype_code, head_dim, block_m, plan["keys"], causal, plan["key_table"])
+
+
 def instance_name(dtype_code, head_dim, block_m, block_n, causal, key_table):
-    """Mangled name of the attn_fwd_kernel instance a launch with these tiles runs (the C ABI's
-    choice: block_m -> 1, 2, 4 or 8 waves of 32 rows, block_n -> 32, 64 or 128 keys; the key-norm
+    """Mangled name of the attn_fwd_kernel instance for these tiles (the C ABI's
+    choice where the general kernel runs: block_m -> 1, 2, 4 or 8 waves of 32 rows, block_n -> 32, 64 or 128 keys; the key-norm
     instance, VARIANT 4, only at the default configuration when the table is in use)."""
     from fa2.kernel import _default_config
 
@@ -123,13 +134,21 @@ def main():
                 lambda: attention(q, k, v, causal=causal, block_m=bm, block_n=bn), args.sustained,
                 flops)
             print(f"sustained block_m={bm} block_n={bn} done", flush=True)
+    from ablation import launch_plan
+    from fa2.kernel import _cu_count, should_pack_gqa
+
     resources = load_resources()
-    key_table = (_lib.workspace_bytes_for(B, H_q, k.shape[1], N, k.shape[2], D, q.dtype, causal, 1)
-                 > _lib.workspace_bytes(B, H_q, N, D, 1))
+    H_kv, N_kv, dt = k.shape[1], k.shape[2], _lib.DTYPE_CODE[q.dtype]
+    cus = _cu_count(q.device)
     rows = []
     for (bm, bn), ms in samples.items():
         med = statistics.median(ms)
-        name = instance_name(_lib.DTYPE_CODE[q.dtype], D, bm, bn, causal, key_table)
+        splits = 1 if causal else _lib.num_splits(B, H_q, H_kv, N, N_kv, D, causal, bm, bn, cus)
+        ws = _lib.workspace_bytes_for(B, H_q, H_kv, N, N_kv, D, q.dtype, causal, splits)
+        pack = H_q // H_kv if should_pack_gqa(N, H_q // H_kv, bm) else 1
+        plan = launch_plan(B, H_q, H_kv, N, N_kv, D, dt, causal, pack=pack, block_m=bm, block_n=bn,
+                           num_splits=splits, workspace_bytes=ws, cus=cus)
+        name = plan_instance(plan, dt, D, bm, causal)
         rows.append({"block_m": bm, "block_n": bn, "median_ms": med,
                      "tflops": flops / (med * 1e-3) / 1e12, "samples_ms": ms,
                      "kernel": name, "resources": resources.get(name),
