@@ -101,6 +101,79 @@ def test_splitkv_packed_equals_unpacked():
         check_against_oracle(q, k, v, False, ours=packed)
 
 
+def _plan(q, k, pack, splits, block_m=128):
+    """The kernel and split count that the library plans for a full call with `splits` asked for."""
+    from ablation import launch_plan
+    from fa2 import _lib
+
+    B, h_q, n_q, D = q.shape
+    return launch_plan(B, h_q, k.shape[1], n_q, k.shape[2], D, 0, False, pack=pack, block_m=block_m,
+                       num_splits=splits, workspace_bytes=_lib.workspace_bytes(B, h_q, n_q, D, splits))
+
+
+# The calls above run the wave-split kernel where it takes them; the general kernel's own splits are
+# below: at the default tiles with more keys than the wave-split rule takes (a ragged last tile), and on
+# the shapes above with rows per program that keep them off it.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("splits,run", [(2, 2), (3, 3), (5, 5), (16, 14)])
+def test_general_kernel_splits_match_oracle(dtype, D, splits, run):
+    attention = _attention()
+    q, k, v = make_qkv(2, 8, 2, 130, 4400, D, dtype)
+    for pack in (1, 4):
+        plan = _plan(q, k, pack, splits)
+        assert plan["kernel"] == "fa2::attn_fwd_kernel"
+        assert plan["splits"] == (12 if D == 16 and splits == 16 else run)  # 35 tiles of 128 keys: 12 of 3
+    out, lse = attention(q, k, v, causal=False, num_splits=splits, return_lse=True)
+    check_against_oracle(q, k, v, False, ours=out)
+    assert_lse(lse, q, k, False)
+    _, lse1 = attention(q, k, v, causal=False, num_splits=1, return_lse=True)
+    assert (lse - lse1).abs().max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [16, 64, 128])
+@pytest.mark.parametrize("block_m,pack_gqa", [(127, False), (96, True), (112, True)])
+@pytest.mark.parametrize("N_q,N_kv", [(1, 1000), (7, 300), (64, 2048), (130, 777)])
+def test_other_tiles_split_in_the_general_kernel(dtype, D, block_m, pack_gqa, N_q, N_kv):
+    attention = _attention()
+    q, k, v = make_qkv(2, 8, 2, N_q, N_kv, D, dtype)
+    for splits in (2, 5):
+        plan = _plan(q, k, 4 if pack_gqa else 1, splits, block_m)
+        assert plan["kernel"] == "fa2::attn_fwd_kernel" and plan["splits"] > 1
+        out, lse = attention(q, k, v, causal=False, num_splits=splits, return_lse=True, block_m=block_m,
+                             pack_gqa=pack_gqa)
+        check_against_oracle(q, k, v, False, ours=out)
+        assert_lse(lse, q, k, False)
+
+
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+def test_general_kernel_splits_packed_equal_unpacked(D):
+    """Two launches of the general kernel that differ (the wave-split kernel ignores the packing)."""
+    attention = _attention()
+    q, k, v = make_qkv(2, 32, 8, 130, 4400, D, torch.float16)
+    for splits in (4, None):
+        n = splits or 4
+        plans = [_plan(q, k, pack, n) for pack in (1, 4)]
+        assert all(p["kernel"] == "fa2::attn_fwd_kernel" and p["splits"] == 4 for p in plans)
+        assert plans[0]["grid"] != plans[1]["grid"]
+        packed = attention(q, k, v, causal=False, pack_gqa=True, num_splits=splits)
+        unpacked = attention(q, k, v, causal=False, pack_gqa=False, num_splits=splits)
+        assert torch.equal(packed, unpacked)
+        check_against_oracle(q, k, v, False, ours=packed)
+
+
+def test_general_kernel_splits_strided_and_repeated():
+    attention = _attention()
+    q, k, v = make_qkv(2, 8, 2, 130, 4400, 64, torch.bfloat16)
+    assert _plan(q, k, 1, 8)["kernel"] == "fa2::attn_fwd_kernel"
+    a = attention(q, k, v, causal=False, num_splits=8)
+    assert torch.equal(a, attention(q, k, v, causal=False, num_splits=8))
+    qs, ks, vs = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v))
+    out = attention(qs, ks, vs, causal=False, num_splits=8)
+    assert out.stride() == qs.stride() and torch.equal(out, a)
+
+
 def test_splitkv_more_splits_than_tiles():
     """16 splits of a 2-tile key range run as 2 splits; 1 key runs as 1."""
     attention = _attention()

@@ -233,3 +233,30 @@ def test_one_general_program_for_three_row_tiles(shape, rows):
     assert _kernel(*shape) == rows
     if rows == 0:
         _only_with_its_splits(shape)
+
+
+# Which kernel the default-tile calls of the GPU tests run (tests/test_gpu_wavesplit.py,
+# tests/test_gpu_splitkv.py), so that a change of the rule cannot take them off it unseen: rows per
+# wave-split workgroup and whether its splits merge, per head_dim
+@needs_ablate
+@pytest.mark.parametrize("shape,causal,want", [
+    ((2, 8, 2, 1, 129), False, {16: (32, 0), 64: (32, 0), 128: (32, 0)}),
+    ((2, 6, 2, 11, 193), False, {D: (32, 0) for D in (16, 32, 64, 128)}),
+    ((2, 5, 1, 13, 4100), False, {D: (32, 1) for D in (16, 32, 64, 128)}),
+    ((2, 2, 2, 64, 9000), False, {D: (32, 1) for D in (16, 32, 64, 128)}),
+    ((2, 8, 2, 65, 2048), False, {D: (32, 1) for D in (16, 32, 64, 128)}),
+    ((2, 8, 2, 64, 2048), False, {D: (32, 1) for D in (16, 32, 64, 128)}),
+    ((17, 8, 8, 40, 300), False, {D: (64, 0) for D in (16, 32, 64, 128)}),
+    ((33, 28, 4, 7, 700), False, {D: (64, 0) for D in (16, 32, 64, 128)}),
+    ((8, 28, 4, 40, 6200), False, {16: (32, 0), 32: (32, 0), 64: (64, 1), 128: (64, 1)}),
+    ((20, 28, 4, 30, 4200), False, {D: (64, 0) for D in (16, 32, 64, 128)}),
+    ((4, 8, 8, 1201, 520), False, {16: (64, 0), 32: (64, 0)}),
+    ((1, 4, 1, 256, 256), True, {D: (32, 0) for D in (16, 32, 64, 128)}),
+    ((2, 16, 16, 520, 520), True, {D: (64, 0) for D in (16, 32, 64, 128)})])
+def test_gpu_tests_reach_the_wave_split_kernel(shape, causal, want):
+    B, h_q, h_kv, n_q, n_kv = shape
+    for D, (rows, merged) in want.items():
+        n = 1 if causal else _lib.num_splits(B, h_q, h_kv, n_q, n_kv, D, causal, 128, 0, 256)
+        plan = _plan(B, h_q, h_kv, n_q, n_kv, D, 0, causal, num_splits=n,
+                     workspace_bytes=_lib.lib().fa2_workspace_bytes(B, h_q, n_q, D, n))
+        assert plan["kernel"] == WAVE_SPLIT and plan["rows"] == rows and (plan["splits"] > 1) == merged, plan
