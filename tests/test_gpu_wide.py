@@ -68,6 +68,50 @@ def test_same_bits_where_the_wide_kernel_runs(dtype, D, table, B, h_q, h_kv, n, 
     _same_as_general(q, k, v, table)
 
 
+@pytest.mark.parametrize("D", [32, 64])
+def test_strided_storage(D):
+    """[B, N, H, D] storage, and K and V as halves of one buffer: the bits of dense tensors."""
+    from ablation import launch_plan
+    from fa2.kernel import attention
+
+    B, h_q, h_kv, n, n_kv = 3, 32, 8, 2047, 1025
+    plan = launch_plan(B, h_q, h_kv, n, n_kv, D, 1, False)
+    assert plan["kernel"] == "fa2::attn_wide_kernel"
+    q, k, v = make_qkv(B, h_q, h_kv, n, n_kv, D, torch.bfloat16)
+    want = _same_as_general(q, k, v)
+    qs, ks, vs = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v))
+    out = attention(qs, ks, vs, causal=False)
+    assert out.stride() == qs.stride() and torch.equal(out, want)
+    kv = torch.stack((k.transpose(1, 2), v.transpose(1, 2)), dim=2)  # [B, N, 2, H, D]
+    ks, vs = kv[:, :, 0].transpose(1, 2), kv[:, :, 1].transpose(1, 2)
+    assert not ks.is_contiguous() and torch.equal(attention(qs, ks, vs, causal=False), want)
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("table", [False, True])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_non_finite_keys_and_values_as_the_general_kernel(D, table, bad):
+    """One element of one key and of one value row, bit for bit the general kernel's outputs."""
+    from fa2 import _lib
+    from fa2.kernel import LOG2E
+
+    B, h_q, h_kv, n, n_kv = 3, 32, 8, 2047, 1025
+    stream = torch.cuda.current_stream().cuda_stream
+    q, k, v = make_qkv(B, h_q, h_kv, n, n_kv, D, torch.float16)
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device=q.device) if table else None
+    for t in (k, v):
+        saved = t[:, 1, 450, 3].clone()
+        t[:, 1, 450, 3] = bad
+        res = []
+        for bm in (128, 127):
+            out = torch.empty_like(q)
+            _lib.attn_fwd_ex(q, k, v, out, False, 1, bm, 0, LOG2E / D ** 0.5, None, 1, ws, stream)
+            res.append(out)
+        assert torch.equal(res[0].isnan(), res[1].isnan()) and res[0].isnan().any() == (t is k or bad != bad)
+        assert torch.equal(res[0].nan_to_num(0.0), res[1].nan_to_num(0.0))
+        t[:, 1, 450, 3] = saved
+
+
 def test_reference_moves_on_every_tile_and_packed_rows():
     from fa2.kernel import attention
 
