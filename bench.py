@@ -473,6 +473,17 @@ def tail_schedule_info(B, H_q, H_kv, N, D, causal):
             "tail_workgroups": out[2].value}
 
 
+def product_plan(q, k, causal):
+    """The launch that attention() makes (ablation.product_plan: the library's planning code in the
+    measurement library, no GPU call), or None where that library is not built."""
+    import ablation
+
+    try:
+        return ablation.product_plan(q, k, causal)
+    except RuntimeError:
+        return None
+
+
 def measured_ceiling(seconds=1.0):
     """The MFMA rate this box sustains under its power limit (triton-fa2-forward_amd/ceiling.py,
     fa2_ablate_mfma_ceiling in the measurement library): bf16 MFMAs on random operands alone, and
@@ -514,7 +525,9 @@ def run(name, steps, warmup, with_cpu, flush_iters, with_sdpa=False, ceiling=Non
     H_kv, N_kv = k.shape[1], k.shape[2]
     key_norm = (_lib.workspace_bytes_for(B, H_q, H_kv, N, N_kv, D, q.dtype, causal, 1)
                 > _lib.workspace_bytes(B, H_q, N, D, 1))
-    kernels = (["fa2::key_norm_kernel"] if key_norm else []) + ["fa2::attn_fwd_kernel"]
+    plan = product_plan(q, k, causal)
+    kernels = (["fa2::key_norm_kernel"] if key_norm else []) + [plan["kernel"] if plan else
+                                                                "the attention kernel"]
 
     settle = settle_clocks(fn)
     with ClockSampler() as timed_clock:
@@ -610,8 +623,7 @@ def run_pack_short(n_q, steps, warmup):
     (bench/bench.py:90-92: bytes of K and V over the time, the bound when N_q is small)."""
     import torch
 
-    from fa2 import _lib
-    from fa2.kernel import _cu_count, attention, should_pack_gqa
+    from fa2.kernel import attention, should_pack_gqa
 
     c = PACK_SHORT
     g = torch.Generator(device="cpu").manual_seed(0)
@@ -630,8 +642,7 @@ def run_pack_short(n_q, steps, warmup):
     med = statistics.median(time_each(fn, steps))
     kv = 2 * k.numel() * k.element_size()
     rate_gbs = kv / (step_ms * 1e-3) / 1e9
-    splits = _lib.num_splits(c["B"], c["H_q"], c["H_kv"], n_q, c["N_kv"], c["D"], False, 128, 64,
-                             _cu_count(q.device))
+    plan = product_plan(q, k, False)
     return {
         "metric": "K/V read rate, few queries against a long K/V (README.md:282-301)",
         "value": round(rate_gbs / 1e3, 3), "unit": "TB/s", "n_gpus": 1, "steps": steps,
@@ -640,7 +651,8 @@ def run_pack_short(n_q, steps, warmup):
         "config": {"workload": f"pack-short: fp16 full B={c['B']} Hq={c['H_q']} Hkv={c['H_kv']} "
                                f"N_q={n_q} N_kv={c['N_kv']} D={c['D']}",
                    "n_q": n_q, "pack_gqa": should_pack_gqa(n_q, c["H_q"] // c["H_kv"], 128),
-                   "num_splits": splits},
+                   "num_splits": plan["splits"] if plan else None,
+                   "kernel": plan["kernel"] if plan else None},
         "us_per_step": round(step_ms * 1e3, 2),
         "per_launch_events_median_us": round(med * 1e3, 2),
         "reference_h100_us": PACK_SHORT_H100_US.get(n_q),

@@ -60,8 +60,8 @@ extern "C" {
  * fa2_ablate_attn_fwd - the forward kernel with the switches in `variant`.
  *
  *   variant  one of the reference's variants (bench/ablation.py:42-53):
- *              0                                          copy (the product kernel, bit for bit
- *                                                         equal to fa2_attn_fwd's launch)
+ *              0                                          copy (bit for bit equal to
+ *                                                         fa2_attn_fwd's launch)
  *              FA2_ABLATE_SCALE_FIRST                     scale_first
  *              FA2_ABLATE_MASK_EVERY_TILE                 mask_every_tile
  *              FA2_ABLATE_SCALE_FIRST | ..._MASK_EVERY_TILE   before_fixes
@@ -75,7 +75,10 @@ extern "C" {
  *            other bit sets are rejected (FA2_EINVAL).
  * The other arguments are fa2_attn_fwd's (include/fa2_fwd.h), with the same checks. Runs at the
  * default configuration (block_m 128, fa2_default_config's block_n), without split-KV, the
- * log-sum-exp or the key-norm table: variant 0 is exactly fa2_attn_fwd's kernel.
+ * log-sum-exp or the key-norm table. Variant 0 runs fa2_attn_fwd's kernel, except where that is the
+ * wide kernel, which has no instance here: the general kernel, with the same bits. Variant
+ * FA2_ABLATE_MASK_EVERY_TILE follows the choice of the wave-split kernel too; every other variant is
+ * the general kernel's (fa2_ablate_plan tells what fa2_attn_fwd runs).
  */
 FA2_API int fa2_ablate_attn_fwd(const void* q, const void* k, const void* v, void* out,
                                 const int64_t q_stride[4], const int64_t k_stride[4],
@@ -88,14 +91,14 @@ FA2_API int fa2_ablate_attn_fwd(const void* q, const void* k, const void* v, voi
 #define FA2_ABLATE_TIMELINE_WORDS 6
 
 /*
- * fa2_ablate_timeline - the product kernel (variant 0, same output bit for bit) with a timeline,
- * in the product's schedule (its dynamic tail included): the workgroup that runs program b (its
+ * fa2_ablate_timeline - the general kernel (same output bit for bit) with a timeline, in the
+ * product's schedule of it (its dynamic tail included): the workgroup that runs program b (its
  * place in the static order) writes FA2_ABLATE_TIMELINE_WORDS uint64 at records[6 b ...]:
  *   [0] entry, [1] prologue done (Q and the first K/V tiles in, first barrier passed),
  *   [2] tile loop done, [3] stores done (after a wait for them): s_memrealtime, 100 MHz;
  *   [4] the workgroup's K/V tile count;
  *   [5] XCC_ID << 32 | HW_ID (hardware ids of the wave that wrote: CU, shader array, engine).
- * It waits for its stores before the last stamp, which the product does not do. No counterpart
+ * It waits for its stores before the last stamp, which the kernel itself does not do. No counterpart
  * in the reference (its profiling used Nsight); a measurement tool for the schedule of short
  * grids. records: device memory, 8-byte aligned, at least 6 x programs words (record_words),
  * where programs = ceil(n_q * pack / 128) * batch * h_q / pack; else FA2_EINVAL, no launch.

@@ -590,6 +590,28 @@ def test_record_and_occupancy_of_the_wave_split_and_wide_kernels():
 
 @needs_lib
 @needs_ablate
+def test_bench_names_the_kernel_attention_runs():
+    """bench.py's lines name the kernel and the split count of the launch that attention() makes."""
+    import bench
+
+    want = {"C2": ("attn_fwd_kernel", False), "C3": ("attn_fwd_kernel", True),
+            "C4": ("attn_wide_kernel", True), "C5": ("attn_fwd_kernel", False)}
+    for cfg, (kernel, table) in want.items():
+        dt, causal, B, h_q, h_kv, n, d, _, _ = bench.WORKLOADS[cfg]
+        dtype = {"fp16": torch.float16, "bf16": torch.bfloat16}[dt]
+        plan = bench.product_plan(torch.empty(B, h_q, n, d, dtype=dtype), torch.empty(B, h_kv, n, d, dtype=dtype),
+                                  causal)
+        assert plan["kernel"] == "fa2::" + kernel and plan["key_table"] == table, (cfg, plan)
+    c = bench.PACK_SHORT
+    k = torch.empty(c["B"], c["H_kv"], c["N_kv"], c["D"], dtype=torch.float16)
+    for n_q, kernel, splits in ((1, "wave_split", 2), (16, "wave_split", 1), (128, "fwd", 1)):
+        plan = bench.product_plan(torch.empty(c["B"], c["H_q"], n_q, c["D"], dtype=torch.float16), k, False)
+        assert plan["kernel"] == f"fa2::attn_{kernel}_kernel", (n_q, plan)
+        assert plan["splits"] == splits, (n_q, plan)
+
+
+@needs_lib
+@needs_ablate
 def test_sweep_names_the_kernel_a_call_runs():
     import sweep
     from ablation import launch_plan

@@ -11,7 +11,7 @@ Every variant is the product's kernel template instantiated with VARIANT bits
 (include/fa2_ablate.h), loaded from the measurement library libfa2_ablate.so, which fa2.kernel
 never loads. The reference's variants (bench/ablation.py:1-20, 42-53):
 
-  copy             no switch: the product kernel, bit for bit the launch of fa2_attn_fwd
+  copy             no switch: bit for bit the launch of fa2_attn_fwd (see below for its kernel)
   scale_first      multiply every score by the scale, then subtract the row max
   mask_every_tile  apply the mask on every K/V tile, not only where needed
   before_fixes     both of the above
@@ -39,6 +39,12 @@ and clock drift hits all variants alike. The table gives each variant's median o
 spread of its rounds, and the change against `copy`. `attention()` is the shipped call on the same
 inputs; on long bf16 problems it adds the key-norm pass and that instance of the kernel (C3), which
 the variants do not have, so the deltas are taken against `copy`, not against it.
+
+The variants are instances of the general kernel, attn_fwd_kernel. Where fa2_attn_fwd runs the wide
+kernel (C4), `copy` is the general kernel with the same bits, so the table says what the general kernel
+spends on that shape, not what attention() does. Where fa2_attn_fwd runs the wave-split kernel, `copy` and
+`mask_every_tile` are that kernel, the other variants are not, and the deltas are taken against
+`general`, the general kernel at 127 rows a program. The table's header names attention()'s kernel.
 
 With --sustained, each variant then also runs alone, back to back, with amdsmi sampling the clock
 and the socket power (sustained_run): the chip holds its power near the limit by lowering the
@@ -126,6 +132,23 @@ def launch_plan(B, H_q, H_kv, N_q, N_kv, D, dtype_code, causal, *, pack=1, block
                            f"{lib.fa2_ablate_last_error().decode(errors='replace')}")
     return {"kernel": KERNELS[info[0]], "rows": info[1], "keys": info[2], "splits": info[3],
             "split_tiles": info[4], "grid": info[5], "key_table": bool(info[6])}
+
+
+def product_plan(q, k, causal, block_m=128, block_n=0):
+    """launch_plan of attention(q, k, ..., causal) on q's device at these tiles: its own packing, split
+    count and workspace."""
+    from fa2 import _lib
+    from fa2.kernel import _cu_count, should_pack_gqa
+
+    B, H_q, N_q, D = q.shape
+    H_kv, N_kv = k.shape[1], k.shape[2]
+    cus = _cu_count(q.device) if q.is_cuda else 256
+    splits = 1 if causal else _lib.num_splits(B, H_q, H_kv, N_q, N_kv, D, causal, block_m, block_n, cus)
+    return launch_plan(B, H_q, H_kv, N_q, N_kv, D, _lib.DTYPE_CODE[q.dtype], causal,
+                       pack=H_q // H_kv if should_pack_gqa(N_q, H_q // H_kv, block_m) else 1,
+                       block_m=block_m, block_n=block_n, num_splits=splits, cus=cus,
+                       workspace_bytes=_lib.workspace_bytes_for(B, H_q, H_kv, N_q, N_kv, D, q.dtype,
+                                                                causal, splits))
 
 
 def variant_bits(switches):
@@ -252,6 +275,7 @@ def measure_shape(args, N):
     import torch
 
     import bench
+    from fa2 import _lib
     from fa2.kernel import attention
 
     dtype = {"fp16": torch.float16, "bf16": torch.bfloat16}[args.dtype]
@@ -264,7 +288,16 @@ def measure_shape(args, N):
 
     product = table_free_launch(q, k, v, causal, block_m=128)
     shipped = attention(q, k, v, causal=causal)
+    plan = product_plan(q, k, causal)
+    # which kernel `copy` runs: without the key-norm table, which the variants never have
+    free = launch_plan(*q.shape[:2], k.shape[1], N, N, args.head_dim, _lib.DTYPE_CODE[dtype], causal)
+    print(f"attention() runs {plan['kernel']}"
+          + (" with the key-norm table" if plan["key_table"] else "") + f", {plan['rows']} rows a workgroup")
     launchers = {"attention()": lambda: attention(q, k, v, causal=causal)}
+    base_name = "copy"
+    if free["kernel"] == KERNELS[1]:
+        base_name = "general"
+        launchers[base_name] = lambda: table_free_launch(q, k, v, causal)
     outputs = {}
     group = args.hq // args.hkv
     for name in args.variants:
@@ -288,14 +321,14 @@ def measure_shape(args, N):
 
     bench.settle_clocks(launchers["copy"] if "copy" in launchers else launchers["attention()"])
     per_round = interleaved_rounds(launchers, args.rounds, args.steps, args.warmup)
-    base = statistics.median(per_round["copy"]) if "copy" in per_round else None
+    base = statistics.median(per_round[base_name]) if base_name in per_round else None
     sustained = {name: sustained_run(fn, args.sustained, flops) for name, fn in launchers.items()} \
         if args.sustained > 0 else {}
     rows = []
     for name, ms in per_round.items():
         med = statistics.median(ms)
         rows.append({"variant": name, "ms": med, "min_ms": min(ms), "max_ms": max(ms),
-                     "vs_copy": (med / base - 1.0) if base else None,
+                     "vs_copy": (med / base - 1.0) if base else None, "base": base_name,
                      "tflops": flops / (med * 1e-3) / 1e12, **checks.get(name, {}),
                      **({"sustained": sustained[name]} if name in sustained else {})})
     del q, k, v, product, shipped, outputs
@@ -308,7 +341,8 @@ def print_table(args, N, rows):
              f"{'full' if args.full else 'causal'}" + (f" inputs x{args.input_scale}" if args.input_scale != 1 else ""))
     print(f"\n{shape}: {args.rounds} rounds of {args.steps} back-to-back launches per variant")
     sus = all("sustained" in r for r in rows)
-    print("| variant | ms per launch (median; min-max over rounds) | vs copy | TFLOP/s | output vs product |"
+    base = rows[0]["base"]
+    print(f"| variant | ms per launch (median; min-max over rounds) | vs {base} | TFLOP/s | output vs product |"
           + (f" alone for {args.sustained:g} s: TFLOP/s | sclk MHz | power W | TFLOP/s per GHz |" if sus else ""))
     print("|---|---|---|---|---|" + ("---|---|---|---|" if sus else ""))
     for r in rows:
@@ -318,7 +352,7 @@ def print_table(args, N, rows):
             out = f"max diff {r['max_abs_diff']:.2e}"
         else:
             out = ""
-        vs = "" if r["vs_copy"] is None or r["variant"] == "copy" else f"{r['vs_copy']:+.1%}"
+        vs = "" if r["vs_copy"] is None or r["variant"] == base else f"{r['vs_copy']:+.1%}"
         extra = ""
         if sus:
             su = r["sustained"]

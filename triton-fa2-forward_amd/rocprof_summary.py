@@ -10,12 +10,14 @@ profile_configs.sh runs, per config, in runs of their own (one counter group per
   <root>/<cfg>_write   rocprofv3 --pmc WRITE_SIZE         1 GiB device copy for the calibration)
   <root>/<cfg>_sq      rocprofv3 --pmc SQ_WAVES SQ_INSTS_MFMA ... GRBM_GUI_ACTIVE
   <root>/<cfg>_util    rocprofv3 --pmc SQ_LDS_IDX_ACTIVE SQ_ACTIVE_INST_VALU ... GRBM_GUI_ACTIVE
-and this module writes, from those CSVs and the bench.py line in <root>/<cfg>_trace.log:
+and, for any other call given as NAME=SHAPE (profile_target.py --shape), the same with a trace over 200
+calls of profile_target.py. This module writes, from those CSVs and the bench.py line in <root>/<cfg>_trace.log:
   profiles/attn_fwd_kernel_<cfg>_kernel_trace.md      per-kernel statistics and the timed steps
   profiles/attn_fwd_kernel_<cfg>_l2_miss_traffic.md   bytes that left L2 per launch
   profiles/attn_fwd_kernel_<cfg>_sq_counters.md       instruction mix, MFMA busy, bank conflicts
   profiles/attn_fwd_kernel_utilisation_counters.md    per-unit busy fractions, all configs
   profiles/l2_miss_traffic.json                        the traffic figures bench.py reports
+  profiles/shape_<name>.md                             --shapes: one call's kernels, traffic and counters
 and, from bench.py's JSON lines (--bench-log: `bench.py --all --sdpa --no-cpu-baseline` then
 `bench.py --pack-short --no-cpu-baseline`, appended to one log), profiles/bench_all_configs.md.
 
@@ -36,7 +38,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 PROFILES = os.path.join(ROOT, "profiles")
 
-ATTN = "attn_fwd_kernel"
+# the attention kernels, by a part of their names; the split-KV merge
+ATTN = ("attn_fwd_kernel", "attn_wave_split_kernel", "attn_wide_kernel")
+COMBINE = "attn_combine_kernel"
 KEY_NORM = "key_norm_kernel"
 COPY = "copyBuffer"
 COPY_KIB = 1 << 20   # profile_target.py --copy-mib 1024: 1 GiB read and 1 GiB written
@@ -90,10 +94,20 @@ def kernel_stats(directory):
              float(r["Percentage"])) for r in read_rows(find_csv(directory, "kernel_stats.csv"))]
 
 
+def named(kernel, name_part):
+    """Whether a kernel's name contains name_part, or one of them."""
+    return any(p in kernel for p in ((name_part,) if isinstance(name_part, str) else name_part))
+
+
+def title(kernel):
+    """fa2::<kernel> of a traced kernel's full name."""
+    return "fa2::" + next((p for p in ATTN if p in kernel), ATTN[0])
+
+
 def dispatches(directory, name_part):
     """[(start ns, end ns)] of the dispatches whose kernel name contains name_part, in time order,
     from *kernel_trace.csv."""
-    rows = [r for r in read_rows(find_csv(directory, "kernel_trace.csv")) if name_part in r["Kernel_Name"]]
+    rows = [r for r in read_rows(find_csv(directory, "kernel_trace.csv")) if named(r["Kernel_Name"], name_part)]
     out = [(int(r["Start_Timestamp"]), int(r["End_Timestamp"])) for r in rows]
     return sorted(out)
 
@@ -111,7 +125,7 @@ def pmc(directory):
 
 def values(disp, name_part, counter):
     """The counter's value of every dispatch of a kernel, in dispatch order."""
-    return [d[counter] for d in disp.values() if name_part in d["kernel"] and counter in d]
+    return [d[counter] for d in disp.values() if named(d["kernel"], name_part) and counter in d]
 
 
 def bench_line(log_path):
@@ -167,7 +181,7 @@ def utilisation(c):
 
 def first_attn(disp):
     for d in disp.values():
-        if ATTN in d["kernel"]:
+        if named(d["kernel"], ATTN):
             return d
     raise ValueError("no attention dispatch in the counter run")
 
@@ -180,8 +194,8 @@ def write_trace(root, cfg, out_dir):
     d = os.path.join(root, f"{cfg}_trace")
     stats = kernel_stats(d)
     b = bench_line(d + ".log")
-    ours = [s for s in stats if ATTN in s[0]]
-    lines = [f"# Kernel trace: fa2::attn_fwd_kernel on {cfg}"
+    ours = [s for s in stats if named(s[0], ATTN)]
+    lines = [f"# Kernel trace: {title(ours[0][0] if ours else '')} on {cfg}"
              + (f" ({b['config']['workload']})" if b else ""), "",
              "Command (run from the repository root on the MI355X box, TMPDIR=/tmp):", "", "```",
              commands(root, cfg)["trace"], "```", "",
@@ -232,7 +246,7 @@ def write_traffic(root, cfg, out_dir, json_path, label):
     except (FileNotFoundError, statistics.StatisticsError):
         pass
     cmd = commands(root, cfg)
-    lines = [f"# L2-miss traffic: fa2::attn_fwd_kernel on {cfg}", "",
+    lines = [f"# L2-miss traffic: {title(first_attn(fetch)['kernel'])} on {cfg}", "",
              "FETCH_SIZE and WRITE_SIZE count the bytes of requests that leave the L2 (TCC); Infinity "
              "Cache (MALL) hits count as well, so the DRAM traffic is at most these figures.", "",
              "Commands (each counter in its own run, TMPDIR=/tmp):", "", "```", cmd["fetch"], cmd["write"],
@@ -260,12 +274,13 @@ def write_traffic(root, cfg, out_dir, json_path, label):
     path = os.path.join(out_dir, f"attn_fwd_kernel_{cfg}_l2_miss_traffic.md")
     with open(path, "w") as f:
         f.write("\n".join(lines))
-    j = {"about": "bytes per launch of fa2::attn_fwd_kernel that left L2 (rocprofv3 FETCH_SIZE + "
-                  "WRITE_SIZE, copy-calibrated; Infinity Cache hits included)", "configs": {}}
+    j = {"configs": {}}
     if os.path.exists(json_path):
         with open(json_path) as f:
             j = json.load(f)
-    j["configs"][cfg] = {"bytes": t["bytes"], "fetch_kib": t["fetch_kib"], "write_kib": t["write_kib"],
+    j = {"about": "bytes per launch of the attention kernel that left L2 (rocprofv3 FETCH_SIZE + "
+                  "WRITE_SIZE, copy-calibrated; Infinity Cache hits included)", "configs": j["configs"]}
+    j["configs"][cfg] = {"kernel": title(first_attn(fetch)["kernel"]), "bytes": t["bytes"], "fetch_kib": t["fetch_kib"], "write_kib": t["write_kib"],
                          "fetch_scale": t["fetch_scale"], "write_scale": t["write_scale"],
                          "kernel_build": label, "algorithmic_bytes": minb,
                          "summary": f"profiles/attn_fwd_kernel_{cfg}_l2_miss_traffic.md"}
@@ -276,7 +291,7 @@ def write_traffic(root, cfg, out_dir, json_path, label):
 
 def write_sq(root, cfg, out_dir):
     first = first_attn(pmc(os.path.join(root, f"{cfg}_sq")))
-    lines = [f"# SQ counters: fa2::attn_fwd_kernel on {cfg} (first profiled launch)", "",
+    lines = [f"# SQ counters: {title(first['kernel'])} on {cfg} (first profiled launch)", "",
              f"Kernel: `{first['kernel']}`", "", "```", commands(root, cfg)["sq"], "```", "",
              "| Counter | Value |", "|---|---|"]
     for n in SQ_COUNTERS:
@@ -307,12 +322,14 @@ def write_util(root, cfgs, out_dir):
     firsts = {c: first_attn(pmc(os.path.join(root, f"{c}_util"))) for c in cfgs}
     u = {c: utilisation(firsts[c]) for c in cfgs}
     cmd = commands(root, "<config>")["util"]
-    lines = [f"# Utilisation counters: fa2::attn_fwd_kernel on {', '.join(cfgs)} (first profiled launch)", "",
+    lines = [f"# Utilisation counters: the attention kernel on {', '.join(cfgs)} (first profiled launch)", "",
              f"One counter pass per config (`<config>` = {', '.join(cfgs)}):", "", "```", cmd, "```", "",
              "Kernel instances (from the runs): "
              + "; ".join(f"{c} `{firsts[c]['kernel']}`" for c in cfgs)
-             + ". Template arguments: <dtype (0 fp16, 1 bf16), head_dim, waves, keys per tile, causal, "
-               "variant>; variant 4 is the instance that reads the key-norm table.", "",
+             + ". Template arguments: attn_fwd_kernel<dtype (0 fp16, 1 bf16), head_dim, waves, keys per tile, "
+               "causal, variant>, variant 4 the instance that reads the key-norm table; "
+               "attn_wave_split_kernel<dtype, head_dim, 32-row waves, keys per tile, causal, variant>; "
+               "attn_wide_kernel<dtype, head_dim, key-norm table>.", "",
              "| Counter (sum over the GPU) | " + " | ".join(cfgs) + " |", "|---|" + "---|" * len(cfgs)]
     for n in ["GRBM_GUI_ACTIVE", "SQ_VALU_MFMA_BUSY_CYCLES", "SQ_VALU_MFMA_COEXEC_CYCLES", "SQ_ACTIVE_INST_VALU",
               "SQ_INSTS_VALU_TRANS_F32", "SQ_LDS_IDX_ACTIVE", "SQ_WAIT_INST_LDS", "SQ_INST_CYCLES_SALU"]:
@@ -334,6 +351,55 @@ def write_util(root, cfgs, out_dir):
     with open(path, "w") as f:
         f.write("\n".join(lines))
     return path, u
+
+
+def write_shape(root, name, out_dir):
+    """profiles/shape_<name>.md: one call's kernels (trace of 200 back-to-back calls), the bytes that left
+    L2 and the per-unit busy fractions of its attention kernel (profile_configs.sh NAME=SHAPE)."""
+    base = os.path.join(root, name)
+    with open(base + "_trace.log") as f:
+        what = next(ln.strip() for ln in f if ln.startswith("profile_target: X:"))
+    spec = what.split()[1].rstrip(",")
+    cmd = commands(root, name)
+    swap = lambda c: c.replace(f"--config {name}", f"--shape {spec}")  # noqa: E731
+    trace = (f"rocprofv3 --kernel-trace --stats --output-format csv -d {root}/{name}_trace -o trace -- python3 "
+             f"triton-fa2-forward_amd/profile_target.py --shape {spec} --launches 200")
+    fetch, write = pmc(base + "_fetch"), pmc(base + "_write")
+    t, first = traffic(fetch, write), first_attn(pmc(base + "_util"))
+    u, sq = utilisation(first), first_attn(pmc(base + "_sq"))
+    # from the 51st dispatch on: the first ones come from an idle GPU
+    us = {}
+    for part in (ATTN, COMBINE, KEY_NORM):
+        d = dispatches(base + "_trace", part)[50:]
+        if d:
+            us[part] = statistics.fmean(e - s for s, e in d) / 1e3
+    rate = t["bytes"] / (us[ATTN] * 1e-6) / 1e9
+    lines = [f"# {title(first['kernel'])} on {name}", "", f"Call: {spec[2:]} (batch, H_q, H_kv, N_q, N_kv, head_dim, "
+             "causal, dtype, with the log-sum-exp where it says lse), `attention()` with its defaults.", "",
+             "Commands (from the repository root on the MI355X box, TMPDIR=/tmp; one counter group a run):", "",
+             "```", trace, *(swap(cmd[c]) for c in ("fetch", "write", "sq", "util")), "```", "",
+             f"Kernel: `{first['kernel']}`", "", "| reading | value |", "|---|---|",
+             f"| attention kernel, mean of the calls from the 51st on | {us[ATTN]:.1f} us |"]
+    if COMBINE in us:
+        lines.append(f"| split-KV merge | {us[COMBINE]:.1f} us |")
+    if KEY_NORM in us:
+        lines.append(f"| key-norm pass | {us[KEY_NORM]:.1f} us |")
+    lines += [f"| bytes past L2 per launch (copy-calibrated FETCH_SIZE + WRITE_SIZE) | {t['bytes'] / 2**20:.1f} MiB |",
+              f"| rate past L2 | {rate:.0f} GB/s |",
+              f"| waves | {sq['SQ_WAVES']:.0f} |",
+              f"| VALU instructions per MFMA | {sq['SQ_INSTS_VALU'] / sq['SQ_INSTS_MFMA']:.2f} |",
+              f"| matrix cores busy | {100 * u['mfma_busy']:.1f}% |",
+              f"| VALU busy per SIMD | {100 * u['valu_busy']:.1f}% |",
+              f"| share of MFMA cycles with VALU work beside them | {100 * u['mfma_with_valu']:.1f}% |",
+              f"| LDS busy | {100 * u['lds_busy']:.1f}% |",
+              f"| LDS bank conflict cycles | {sq['SQ_LDS_BANK_CONFLICT']:.0f} |", "",
+              "The counter runs are three calls from an idle GPU; their busy fractions are over the kernel's own "
+              "active time.", "",
+              "Made by `python triton-fa2-forward_amd/rocprof_summary.py --shapes " + name + "` from the runs' CSVs.", ""]
+    path = os.path.join(out_dir, f"shape_{name}.md")
+    with open(path, "w") as f:
+        f.write("\n".join(lines))
+    return path
 
 
 def bench_lines(log_path):
@@ -379,12 +445,13 @@ def write_bench(log_path, out_dir):
         L += ["", "Few queries against a long K/V (the reference's README.md:282-301 table; fp16, B 16, "
                   "H 32/8, N_kv 4096, D 128, non-causal; K + V = 256 MiB read once per call):", "",
               "| N_q | us per call | K/V read rate TB/s | frac of 8 TB/s | frac of a streaming read of the "
-              "same size | splits | reference H100 us | speedup |",
-              "|---|---|---|---|---|---|---|---|"]
+              "same size | kernel | splits | reference H100 us | speedup |",
+              "|---|---|---|---|---|---|---|---|---|"]
         for b in short:
             r = b["roofline"]
             L.append(f"| {b['config']['n_q']} | {b['us_per_step']} | {b['value']} | {r['frac']} | "
-                     f"{r.get('frac_of_measured_read_rate', '-')} | {b['config']['num_splits']} | "
+                     f"{r.get('frac_of_measured_read_rate', '-')} | "
+                     f"{(b['config'].get('kernel') or '-').replace('fa2::', '')} | {b['config']['num_splits']} | "
                      f"{b.get('reference_h100_us', '-')} | {b.get('vs_reference_h100', '-')}x |")
     L += ["", "Made by `python triton-fa2-forward_amd/rocprof_summary.py --bench-log <log>` from the "
               "runs' JSON lines.", ""]
@@ -397,7 +464,8 @@ def write_bench(log_path, out_dir):
 def main():
     ap = argparse.ArgumentParser(description=__doc__.splitlines()[0])
     ap.add_argument("--root", default="gpurun_out/prof", help="profile_configs.sh's output folder")
-    ap.add_argument("--configs", nargs="+", default=["C3", "C2", "C4", "C5"])
+    ap.add_argument("--configs", nargs="*", default=["C3", "C2", "C4", "C5"])
+    ap.add_argument("--shapes", nargs="*", default=[], help="names of profile_configs.sh's NAME=SHAPE runs")
     ap.add_argument("--out", default=PROFILES)
     ap.add_argument("--json", default=os.path.join(PROFILES, "l2_miss_traffic.json"))
     ap.add_argument("--label", default="current", help="kernel_build label in the JSON")
@@ -408,6 +476,8 @@ def main():
     if args.bench_log:
         print(write_bench(args.bench_log, args.out))
     os.makedirs(args.out, exist_ok=True)
+    for name in args.shapes:
+        print(write_shape(args.root, name, args.out))
     for cfg in args.configs:
         if "trace" in args.parts:
             print(write_trace(args.root, cfg, args.out))
@@ -416,7 +486,7 @@ def main():
             print(path, t["bytes"])
         if "sq" in args.parts:
             print(write_sq(args.root, cfg, args.out))
-    if "util" in args.parts:
+    if "util" in args.parts and args.configs:
         print(write_util(args.root, args.configs, args.out)[0])
 
 

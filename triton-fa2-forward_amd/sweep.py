@@ -134,21 +134,14 @@ def main():
                 lambda: attention(q, k, v, causal=causal, block_m=bm, block_n=bn), args.sustained,
                 flops)
             print(f"sustained block_m={bm} block_n={bn} done", flush=True)
-    from ablation import launch_plan
-    from fa2.kernel import _cu_count, should_pack_gqa
+    from ablation import product_plan
 
     resources = load_resources()
-    H_kv, N_kv, dt = k.shape[1], k.shape[2], _lib.DTYPE_CODE[q.dtype]
-    cus = _cu_count(q.device)
     rows = []
     for (bm, bn), ms in samples.items():
         med = statistics.median(ms)
-        splits = 1 if causal else _lib.num_splits(B, H_q, H_kv, N, N_kv, D, causal, bm, bn, cus)
-        ws = _lib.workspace_bytes_for(B, H_q, H_kv, N, N_kv, D, q.dtype, causal, splits)
-        pack = H_q // H_kv if should_pack_gqa(N, H_q // H_kv, bm) else 1
-        plan = launch_plan(B, H_q, H_kv, N, N_kv, D, dt, causal, pack=pack, block_m=bm, block_n=bn,
-                           num_splits=splits, workspace_bytes=ws, cus=cus)
-        name = plan_instance(plan, dt, D, bm, causal)
+        plan = product_plan(q, k, causal, bm, bn)
+        name = plan_instance(plan, _lib.DTYPE_CODE[q.dtype], D, bm, causal)
         rows.append({"block_m": bm, "block_n": bn, "median_ms": med,
                      "tflops": flops / (med * 1e-3) / 1e12, "samples_ms": ms,
                      "kernel": name, "resources": resources.get(name),

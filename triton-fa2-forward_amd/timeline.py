@@ -2,7 +2,8 @@
 
     python triton-fa2-forward_amd/timeline.py --config C5 [--launches 20] [--csv out.csv]
 
-Runs the product kernel through the measurement library's timeline instance
+Runs the general kernel (attn_fwd_kernel: what attention() runs on C2, C3 and C5; the wide kernel it runs
+on C4 has the same bits and no timeline instance) through the measurement library's timeline instance
 (fa2_ablate_timeline, include/fa2_ablate.h): the same attention bit for bit, with every
 workgroup recording s_memrealtime (100 MHz) at entry, when its prologue is done (Q and the first
 K/V tiles in, first barrier passed), when its tile loop is done and when its stores are done, plus
@@ -14,8 +15,8 @@ its K/V tile count and the hardware ids of the CU it ran on. The summary of the 
   * when the second-round workgroups (those that waited for a free slot) started and ended;
   * per XCD: workgroups, tiles of work and when its last workgroup ended.
 
-The timeline instance waits for its stores before the last stamp, which the product kernel does
-not; its launch is therefore slightly longer than the product's (reported beside it).
+The timeline instance waits for its stores before the last stamp, which the kernel itself does
+not; its launch is therefore slightly longer than the kernel's (reported beside it).
 """
 
 import argparse
@@ -38,10 +39,10 @@ Commands (committed code only; the timeline instance is in libfa2_ablate.so):
     python triton-fa2-forward_amd/timeline.py --config {cfg} --csv {csv}
     python triton-fa2-forward_amd/timeline.py --config {cfg} --from-csv {csv} --md profiles/timeline_{cfg}.md
 
-Every workgroup of the timeline instance (the product kernel, bit for bit, plus s_memrealtime
+Every workgroup of the timeline instance (the general kernel, bit for bit, plus s_memrealtime
 stamps at 100 MHz) records entry, prologue done (Q and the first K/V tiles in, first barrier),
 tile loop done and stores done, its K/V tile count and the hardware id of its CU. It waits for its
-stores before the last stamp, which the product kernel does not, so its span is a little longer.
+stores before the last stamp, which the kernel itself does not, so its span is a little longer.
 """
 TICK_US = 0.01     # s_memrealtime runs at 100 MHz
 
@@ -204,7 +205,7 @@ def main():
     import torch
 
     import bench
-    from ablation import table_free_launch
+    from ablation import KERNELS, attention_ablate, product_plan, table_free_launch
 
     q, k, v, causal = bench.make_inputs(args.config, "cuda")
     B, H_q, N, D = q.shape
@@ -213,20 +214,20 @@ def main():
     bench.settle_clocks(lambda: table_free_launch(q, k, v, causal), min_ms=500.0)
     recs, out = run_timeline(q, k, v, causal, args.launches)
     if not torch.equal(out, product):
-        raise SystemExit("the timeline instance's output differs from the product kernel's")
-    # the product kernel alone, back to back into one preallocated output (fa2_attn_fwd)
-    from fa2 import _lib
-    from fa2.kernel import LOG2E
+        raise SystemExit("the timeline instance's output differs from the general kernel's")
+    # the general kernel alone, back to back (the measurement library's copy, without the key-norm table),
+    # and attention(), whatever it runs
+    from fa2.kernel import attention
 
-    o = torch.empty_like(q)
-    stream = torch.cuda.current_stream().cuda_stream
-    scale = LOG2E / math.sqrt(D)
     steps = 200
-    prod_ms, _ = bench.time_steps(lambda: _lib.attn_fwd(q, k, v, o, causal, 1, 128, 0, scale, stream),
-                                  steps, 5)
+    plan = product_plan(q, k, causal)
+    copy_ms, _ = bench.time_steps(lambda: attention_ablate(q, k, v, causal=causal), steps, 5)
+    prod_ms, _ = bench.time_steps(lambda: attention(q, k, v, causal=causal), steps, 5)
     rows, text = summarize(recs, flops)
-    head = (f"{bench.describe(args.config)}; output bit-exact with the product kernel; product kernel "
-            f"back to back {prod_ms / steps * 1e3:.2f} us per launch")
+    head = (f"{bench.describe(args.config)}; output bit-exact with the general kernel, {KERNELS[0]}, back to "
+            f"back {copy_ms / steps * 1e3:.2f} us per launch; attention() runs {plan['kernel']}"
+            + (" with the key-norm pass" if plan["key_table"] else "")
+            + f", {prod_ms / steps * 1e3:.2f} us per call")
     print(head)
     print(text)
     if args.csv:
