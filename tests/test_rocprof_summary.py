@@ -33,6 +33,14 @@ def test_copy_calibration_and_l2_miss_bytes():
     assert abs(t["bytes"] - 334054699) <= 1      # the committed figure for this run
 
 
+def test_the_calibration_copy_is_the_largest_copy():
+    """Inputs of a few KiB reach the GPU through the same copy kernel, before the calibration copy."""
+    disp = rs.pmc(os.path.join(FIX, "C3_fetch"))
+    want = rs.copy_reading(disp, "FETCH_SIZE")
+    small = {0: {"kernel": "__amd_rocclr_copyBuffer", "FETCH_SIZE": 6.5}}
+    assert rs.copy_reading({**small, **disp}, "FETCH_SIZE") == want > 1e5
+
+
 def test_key_norm_dispatches_are_not_attention():
     fetch = rs.pmc(os.path.join(FIX, "C3_fetch"))
     assert len(rs.values(fetch, rs.KEY_NORM, "FETCH_SIZE")) == 3

@@ -8,17 +8,25 @@ Design decisions of a few percent (a schedule rule, a register budget, a tail po
 by timing two builds of the same sources on the same box, in one process: clocks on MI355X move
 by several percent between boxes and over minutes under the power limit, so numbers from two
 runs do not compare. Each library is loaded from its own path (ctypes), called as attention()
-calls the product (fa2_attn_fwd_ex with a workspace of fa2_workspace_bytes_for bytes: the
-key-norm table where it pays, default tiles, no split-KV), and the outputs of all libraries are
-compared bit for bit with the first one's before and after timing (a schedule change must not
-change a result). Clocks are settled once (bench.settle_clocks); then, round after round, every
+calls the product (fa2_attn_fwd_ex at the default tiles with the library's own packing, split count and
+workspace of fa2_workspace_bytes_for bytes: the key-norm table where it pays), and the outputs of all
+libraries are compared bit for bit with the first one's before and after timing (a schedule change must not
+change a result; another kernel may, by rounding). Clocks are settled once (bench.settle_clocks); then, round after round, every
 library runs W warmups and K launches back to back between one pair of HIP events
 (bench.time_steps), in forward order on even rounds and reverse order on odd rounds, so that
 drift within a round hits all libraries alike. The reference interleaves its variants the same
 way (bench/ablation.py:252-255).
 
+The kernel choice (attn_fwd_host.hpp: kernel_choice, wide_pays) is measured against the general kernel
+alone the same way, over the shapes on both sides of a line:
+
+    python triton-fa2-forward_amd/csrc/build.py --variant general -D FA2_GENERAL_ONLY=1
+    python triton-fa2-forward_amd/ab.py --libs cur=triton-fa2-forward_amd/fa2/libfa2_fwd.so \\
+        general=triton-fa2-forward_amd/variants/general/libfa2_fwd.so --configs \\
+        X:3:12:12:41x4352:128:0:bf16 X:8:16:16:67x150:64:0:fp16 X:1:32:8:1024:128:1:bf16
+
 Workloads: the BASELINE configs by name (C2..C5), or X:B:Hq:Hkv:N:D:causal:dtype[:scale] for any
-other shape (q, k, v from a CPU generator with seed 0, times scale); a ":nt" suffix gives no
+other shape (q, k, v from a CPU generator with seed 0, times scale), N as N_qxN_kv where they differ; a ":nt" suffix gives no
 workspace (no key-norm table), a ":kt" suffix a workspace with room for the table whatever the
 library's policy says (the table then always runs). A library given as NAME=PATH@kt or @nt
 takes that table mode on every workload, so that one build can be timed with and without the
@@ -86,8 +94,9 @@ def make_workload(spec):
         scale = float(f[8]) if len(f) > 8 else 1.0
         g = torch.Generator(device="cpu").manual_seed(0)
         dtype = {"bf16": torch.bfloat16, "fp16": torch.float16}[dt]
-        q, k, v = ((torch.randn(int(B), int(h), int(n), int(d), generator=g) * scale).to(dtype).cuda()
-                   for h in (hq, hkv, hkv))
+        nq, nkv = n.split("x") if "x" in n else (n, n)
+        q, k, v = ((torch.randn(int(B), int(h), int(m), int(d), generator=g) * scale).to(dtype).cuda()
+                   for h, m in ((hq, nq), (hkv, nkv), (hkv, nkv)))
         return q, k, v, c == "1", table
     q, k, v, causal = bench.make_inputs(base, "cuda")
     return q, k, v, causal, table
@@ -98,14 +107,19 @@ def make_call(h, q, k, v, out, causal, table, block_m=128):
     import torch
 
     from fa2 import _lib
+    from fa2.kernel import _cu_count
 
     B, Hq, Nq, D = q.shape
     Hkv, Nkv = k.shape[1], k.shape[2]
     dt = _lib.DTYPE_CODE[q.dtype]
+    splits = 1 if causal else h.fa2_num_splits(B, Hq, Hkv, Nq, Nkv, D, 0, block_m, 0,
+                                               _cu_count(q.device))
+    pack = Hq // Hkv if h.fa2_should_pack_gqa(Nq, Hq // Hkv, block_m) else 1
+    nb = h.fa2_workspace_bytes(B, Hq, Nq, D, splits)
     if table == "force":   # room for the key-norm table: one float per (batch, kv head, 64 keys)
-        nb = (B * Hkv * ((Nkv + 63) // 64) * 4 + 255) // 256 * 256
-    else:
-        nb = h.fa2_workspace_bytes_for(B, Hq, Hkv, Nq, Nkv, D, dt, int(causal), 1) if table else 0
+        nb += (B * Hkv * ((Nkv + 63) // 64) * 4 + 255) // 256 * 256
+    elif table:
+        nb = h.fa2_workspace_bytes_for(B, Hq, Hkv, Nq, Nkv, D, dt, int(causal), splits)
     ws = torch.empty(max(nb, 1), dtype=torch.uint8, device="cuda")
     strides = [_lib._strides(t) for t in (q, k, v, out)]
     scale = 1.4426950408889634 / math.sqrt(D)
@@ -113,7 +127,7 @@ def make_call(h, q, k, v, out, causal, table, block_m=128):
 
     def fn():
         rc = h.fa2_attn_fwd_ex(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), *strides,
-                               B, Hq, Hkv, Nq, Nkv, D, dt, int(causal), 1, block_m, 0, scale, None, 1,
+                               B, Hq, Hkv, Nq, Nkv, D, dt, int(causal), pack, block_m, 0, scale, None, splits,
                                ws.data_ptr() if nb else None, nb, stream)
         if rc:
             raise RuntimeError(h.fa2_last_error().decode())

@@ -217,6 +217,12 @@ int general_splits(int64_t programs, int64_t n_kv, int32_t bn, int cus) {
   return s;
 }
 
+// 1: no call takes the wave-split or the wide kernel, compile-time so that ab.py can measure the rules
+// below against the general kernel alone.
+#ifndef FA2_GENERAL_ONLY
+#define FA2_GENERAL_ONLY 0
+#endif
+
 // Key ranges of whole tiles that `tiles` are cut into when n are asked for: none is empty.
 int clamp_splits(int64_t tiles, int n) {
   const int64_t per = (tiles + n - 1) / n;
@@ -227,7 +233,7 @@ KernelChoice kernel_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q
                            int32_t head_dim, bool causal, int32_t block_m, int32_t bn, int cus,
                            int num_splits) {
   KernelChoice kc;
-  if (block_m != 128 || bn != default_block_n(head_dim)) return kc;
+  if (FA2_GENERAL_ONLY || block_m != 128 || bn != default_block_n(head_dim)) return kc;
   const int64_t rows = n_q * (h_q / h_kv), units = batch * h_kv;
   if (n_kv <= (head_dim == 128 && (causal || rows > 32) ? 192 : 128)) return kc;
   if (rows > (int64_t(1) << 22) || units > (int64_t(1) << 22)) return kc;  // (products below fit)
@@ -403,7 +409,7 @@ SplitChoice split_choice(int64_t batch, int64_t h_q, int64_t h_kv, int64_t n_q, 
 //     -4..+1%, 10/9 +5..8%, 10/10 -4..-1%, 12/11 0..+6%, 12/12 -6..-2%, 14/13 -3..+2%, 16/15 0..+1%, 16/16
 //     -2..-6%, 22/21 -1%. Two per CU leave one in three places of a CU empty: 4/4 +4..5% (N1024), 0..1%.
 bool wide_pays(int64_t rows, int64_t n_bh, int64_t n_kv, int32_t head_dim, int cus) {
-  if ((head_dim != 32 && head_dim != 64) || n_kv < 1024) return false;
+  if (FA2_GENERAL_ONLY || (head_dim != 32 && head_dim != 64) || n_kv < 1024) return false;
   const int64_t tiles = (rows + fa2::kWideRows - 1) / fa2::kWideRows, general_tiles = (rows + 127) / 128;
   if (tiles * 2 * 100 > general_tiles * 102) return false;
   const int64_t programs = tiles * n_bh;

@@ -3,11 +3,12 @@
 
     python triton-fa2-forward_amd/isa_stats.py                                # bf16 D128 causal, key-norm
     python triton-fa2-forward_amd/isa_stats.py --dtype fp16 --head-dim 64 --full --variant 0
+    python triton-fa2-forward_amd/isa_stats.py --dtype fp16 --head-dim 64 --wide  # C4's: the wide kernel
     python triton-fa2-forward_amd/isa_stats.py --dump kernel.s                # keep the listing
 
 Compiles csrc/attn_fwd_inst.hip for one (dtype, head_dim) pair to gfx950 assembly (hipcc -S,
 device only; no GPU needed) with the library's own flags, takes one instance of
-attn_fwd_kernel<DT, D, waves, block_n, causal, VARIANT>, and prints:
+attn_fwd_kernel<DT, D, waves, block_n, causal, VARIANT> or attn_wide_kernel<DT, D, KB>, and prints:
 
   * its resources from the code object's metadata (VGPRs, AGPRs, SGPRs, spills, LDS);
   * every loop (a backward branch and the blocks it spans), and for the tile loop (the innermost
@@ -142,6 +143,10 @@ def kernel_name(dt, d, waves, block_n, causal, variant):
             f"ELi{variant}EEEvNS_6ParamsE")
 
 
+def wide_kernel_name(dt, d, key_norm):
+    return f"_ZN3fa216attn_wide_kernelILi{dt}ELi{d}ELb{int(key_norm)}EEEvNS_6ParamsE"
+
+
 def compile_listing(dt, d, out_path=None):
     """gfx950 assembly of csrc/attn_fwd_inst.hip for one (dtype, head_dim) pair, with the
     library's flags (csrc/build.py)."""
@@ -211,6 +216,7 @@ def main():
     ap.add_argument("--waves", type=int, default=4)
     ap.add_argument("--block-n", type=int, default=None)
     ap.add_argument("--variant", type=int, default=4, help="0: table-free; 4: key-norm (C3's)")
+    ap.add_argument("--wide", action="store_true", help="attn_wide_kernel (head_dim 32 and 64, full)")
     ap.add_argument("--dump", default=None, help="also keep the listing here")
     args = ap.parse_args()
 
@@ -218,7 +224,8 @@ def main():
 
     dt = {"fp16": 0, "bf16": 1}[args.dtype]
     bn = args.block_n or (128 if args.head_dim == 16 else 64)
-    name = kernel_name(dt, args.head_dim, args.waves, bn, not args.full, args.variant)
+    name = (wide_kernel_name(dt, args.head_dim, args.variant == 4) if args.wide else
+            kernel_name(dt, args.head_dim, args.waves, bn, not args.full, args.variant))
     asm = compile_listing(dt, args.head_dim, args.dump)
     text, _ = report(asm, name)
     print(f"hipcc {' '.join(build.common_flags()[:3])} ... --cuda-device-only -S "
