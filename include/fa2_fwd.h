@@ -97,9 +97,14 @@ FA2_API int fa2_attn_fwd(const void* q, const void* k, const void* v, void* out,
  *              that many pieces of whole K/V tiles (fewer if the key range is shorter), one
  *              workgroup each, and a second kernel merges the pieces. For grids too small
  *              to fill the GPU: few queries against a long K/V. fa2_num_splits() picks it.
- *              At the default tiles (block_m 128), few rows per KV head and small grids run a
- *              kernel whose workgroups share a row's keys among their waves; it takes at most
- *              num_splits pieces, and fewer where those already reach every CU.
+ *              At the default tiles (block_m 128, the default block_n) and without room for
+ *              the key-norm table, few rows per KV head and small grids run a kernel whose
+ *              workgroups share a row's keys among their waves (causal calls too); it takes at
+ *              most num_splits pieces, and fewer where those already reach every CU. Which
+ *              kernel runs depends on the sizes (batch and head counts included), on num_splits
+ *              and on the GPU's CU count, and it adds up a row's keys in an order of its own: the
+ *              same sequence alone and in a batch may differ by rounding. block_m 127 with pack 1
+ *              keeps any call on the general kernel.
  *   workspace  device memory, 256-byte aligned, owned by the caller and untouched until the
  *              launch has run; may be NULL when num_splits == 1. It must hold at least
  *              fa2_workspace_bytes(batch, h_q, n_q, head_dim, num_splits) bytes (the split-KV
@@ -109,6 +114,10 @@ FA2_API int fa2_attn_fwd(const void* q, const void* k, const void* v, void* out,
  *              prove, per row, that later scores cannot pass the row's first-tile max by more
  *              than 15 (fp16) or 32 (bf16) in exp2 units (a weight of at most 2^15 or
  *              2^32), and then skips the per-tile row max.
+ *              The kernel that uses the table is the general one, whatever the size: a caller
+ *              with one large buffer for every call passes as workspace_bytes what
+ *              fa2_workspace_bytes_for() says, not the buffer's size, or its short calls miss
+ *              the kernel for small grids.
  *              Only at the default configuration (block_m <= 128 rounds to 4 waves and the
  *              default block_n); otherwise the room is left unused. Same attention either way
  *              (the same 2x-SDPA accuracy); the bits of rows that skip can differ from a launch
@@ -182,10 +191,9 @@ FA2_API size_t fa2_workspace_bytes_for(int32_t batch, int32_t h_q, int32_t h_kv,
 /*
  * fa2_num_splits - the split count fa2_attn_fwd_ex should use: 1 for causal launches and for
  * grids of at least num_cus workgroups; otherwise the smallest power of two that reaches it,
- * keeping at least 4 K/V tiles per split, at most 16; or more where the kernel for few rows per KV
- * head (at most 64) uses more. The grid it sizes is the
- * smaller of the packed and the unpacked GQA layouts, so the answer does not depend on the
- * packing decision and packed and unpacked launches stay equal bit for bit. Host policy only.
+ * keeping at least 4 K/V tiles per split, at most 16; or more where the kernel for few rows and
+ * small grids (see fa2_attn_fwd_ex) uses more. The grid it sizes is the smaller of the packed and the
+ * unpacked GQA layouts, so the answer does not depend on the packing decision and packed and unpacked launches stay equal bit for bit. Host policy only.
  */
 FA2_API int32_t fa2_num_splits(int32_t batch, int32_t h_q, int32_t h_kv, int32_t n_q, int32_t n_kv,
                                int32_t head_dim, int32_t causal, int32_t block_m, int32_t block_n,

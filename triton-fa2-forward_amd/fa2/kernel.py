@@ -102,6 +102,10 @@ def attention(q, k, v, causal=True, sm_scale=None, block_m=None, block_n=None,
         tiles, few rows per KV head and small grids share a row's keys among a workgroup's waves
         first and take at most this many splits. The pick does not depend on pack_gqa, so packed
         and unpacked results stay equal bit for bit.
+        Which kernel runs depends on the sizes, batch and head counts included, and on the GPU's CU
+        count, so a row's last bits can differ between the same sequence alone and in a batch
+        (block_m=127, pack_gqa=False and num_splits=1 keep a call on the general kernel; long
+        problems add the key-norm table to it, which can change last bits as well).
     return_lse: also return the natural-log log-sum-exp of every row's scaled scores, fp32
         [B, H_q, N_q], i.e. (out, lse).
     """
